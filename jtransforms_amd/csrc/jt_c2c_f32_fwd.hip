@@ -1,0 +1,6 @@
+// The complex engine's FP32 forward transforms.
+#include "jt_fft1d.hpp"
+
+namespace jt {
+JT_C2C_INST(, float, -1)
+}  // namespace jt

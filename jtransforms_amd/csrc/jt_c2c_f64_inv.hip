@@ -1,0 +1,6 @@
+// The complex engine's FP64 backward transforms.
+#include "jt_fft1d.hpp"
+
+namespace jt {
+JT_C2C_INST(, double, 1)
+}  // namespace jt

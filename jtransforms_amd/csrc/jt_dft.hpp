@@ -193,6 +193,60 @@ __device__ __forceinline__ void dft16(cpx<T>* v) {
         for (int p = 0; p < 4; p++) v[m + 4 * p] = t[4 * m + p];
 }
 
+// Composite radix N = A*B with coprime A and B, by the Good-Thomas index maps
+// (no internal twiddles): input (B j1 + A j2) mod N, output k with
+// k mod A = k1 and k mod B = k2.
+template <int R, int DIR, typename T>
+__device__ __forceinline__ void dft(cpx<T>* v);
+
+constexpr int crt_index(int k1, int k2, int A, int B) {
+    int k = k1;
+    while (k % B != k2) k += A;
+    return k;
+}
+template <int A, int B, int DIR, typename T>
+__device__ __forceinline__ void dft_coprime(cpx<T>* v) {
+    cpx<T> u[A * B];
+#pragma unroll
+    for (int j2 = 0; j2 < B; j2++) {
+        cpx<T> a[A];
+#pragma unroll
+        for (int j1 = 0; j1 < A; j1++) a[j1] = v[(B * j1 + A * j2) % (A * B)];
+        dft<A, DIR>(a);
+#pragma unroll
+        for (int k1 = 0; k1 < A; k1++) u[k1 * B + j2] = a[k1];
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < A; k1++) {
+        dft<B, DIR>(u + k1 * B);
+#pragma unroll
+        for (int k2 = 0; k2 < B; k2++) v[crt_index(k1, k2, A, B)] = u[k1 * B + k2];
+    }
+}
+
+// radix 9 = 3 x 3 with internal twiddles exp(DIR*2pi*i*j*k/9)
+template <int DIR, typename T>
+__device__ __forceinline__ void dft9(cpx<T>* v) {
+    const T c1 = T(0.76604444311897803520), s1 = T(DIR) * T(0.64278760968653932632);   // 2pi/9
+    const T c2 = T(0.17364817766693034885), s2 = T(DIR) * T(0.98480775301220805937);   // 4pi/9
+    const T c4 = T(-0.93969262078590838405), s4 = T(DIR) * T(0.34202014332566873304);  // 8pi/9
+#pragma unroll
+    for (int q = 0; q < 3; q++) dft3<DIR>(v[q], v[q + 3], v[q + 6]);
+    // element q + 3m holds k1 = m of column q: times w9^(q m)
+    auto tw = [](cpx<T>& a, T c, T s) { a = {a.x * c - a.y * s, a.x * s + a.y * c}; };
+    tw(v[4], c1, s1);
+    tw(v[5], c2, s2);
+    tw(v[7], c2, s2);
+    tw(v[8], c4, s4);
+#pragma unroll
+    for (int m = 0; m < 3; m++) dft3<DIR>(v[3 * m], v[3 * m + 1], v[3 * m + 2]);
+    // output X_{m + 3p} sits at v[3m + p]; transpose 3x3
+    cpx<T> t;
+    t = v[1]; v[1] = v[3]; v[3] = t;
+    t = v[2]; v[2] = v[6]; v[6] = t;
+    t = v[5]; v[5] = v[7]; v[7] = t;
+}
+
 // Generic in-register DFT dispatch on a compile-time radix.
 template <int R, int DIR, typename T>
 __device__ __forceinline__ void dft(cpx<T>* v) {
@@ -200,8 +254,14 @@ __device__ __forceinline__ void dft(cpx<T>* v) {
     else if constexpr (R == 3) dft3<DIR>(v[0], v[1], v[2]);
     else if constexpr (R == 4) dft4<DIR>(v[0], v[1], v[2], v[3]);
     else if constexpr (R == 5) dft5<DIR>(v[0], v[1], v[2], v[3], v[4]);
+    else if constexpr (R == 6) dft_coprime<2, 3, DIR>(v);
     else if constexpr (R == 7) dft7<DIR>(v);
     else if constexpr (R == 8) dft8<DIR>(v);
+    else if constexpr (R == 9) dft9<DIR>(v);
+    else if constexpr (R == 10) dft_coprime<2, 5, DIR>(v);
+    else if constexpr (R == 12) dft_coprime<4, 3, DIR>(v);
+    else if constexpr (R == 14) dft_coprime<2, 7, DIR>(v);
+    else if constexpr (R == 15) dft_coprime<3, 5, DIR>(v);
     else if constexpr (R == 16) dft16<DIR>(v);
     else static_assert(R == 2, "unsupported radix");
 }

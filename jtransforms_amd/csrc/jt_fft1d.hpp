@@ -6,13 +6,16 @@
 // 117-188) but chosen for the GPU:
 //   TPL   n a power of two in [16, 4096]: compile-time stockham_kernel
 //   GEN   n <= LDS limit with factors in {2,3,5,7,11,13}: generic_kernel
-//   FOUR  smooth n above the LDS limit: n = n1*n2, two LDS passes
+//   FOUR  smooth n above the LDS limit: n = n1*n2, two LDS passes, both over
+//         columns (the first leaves the transpose)
 //   BLUE  any other n: Bluestein chirp-z over a smooth length m >= 2n-1
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <functional>
 #include <memory>
 #include <stdexcept>
 #include <string>
@@ -145,6 +148,35 @@ inline bool mf_radices(int64_t n, std::vector<int>& r) {
     }
 }
 
+// Stages of the runtime-radix kernel: the fewest radices up to 16, among
+// those the smallest sum; odd radices first (their first-stage LDS writes, at
+// stride R, spread over the banks).
+inline std::vector<int> gen_radices(int64_t n) {
+    std::vector<int> best, cur;
+    auto sum = [](const std::vector<int>& v) {
+        int t = 0;
+        for (int x : v) t += x;
+        return t;
+    };
+    std::function<void(int64_t, int)> rec = [&](int64_t r, int most) {
+        if (r == 1) {
+            if (best.empty() || cur.size() < best.size() || (cur.size() == best.size() && sum(cur) < sum(best)))
+                best = cur;
+            return;
+        }
+        if ((int)cur.size() >= GEN_STAGES || (!best.empty() && cur.size() >= best.size())) return;
+        for (int R = most; R >= 2; R--)
+            if (r % R == 0) {
+                cur.push_back(R);
+                rec(r / R, R);
+                cur.pop_back();
+            }
+    };
+    rec(n, 16);
+    std::stable_sort(best.begin(), best.end(), [](int a, int b) { return (a & 1) > (b & 1); });
+    return best;
+}
+
 template <typename T>
 inline int64_t gen_max() { return sizeof(T) == 8 ? 4096 : 8192; }
 
@@ -156,6 +188,23 @@ std::vector<cpx<T>> stage_twiddles(const std::vector<int>& radices, std::vector<
         if (offs) offs->push_back((int)tw.size());
         for (int64_t jm = 0; jm < ns; jm++)
             for (int r = 1; r < R; r++) tw.push_back(expm<T>(jm * r, ns * R));
+        ns *= R;
+    }
+    if (tw.empty()) tw.push_back(cpx<T>{T(1), T(0)});
+    return tw;
+}
+
+// Twiddles of the runtime-radix kernel: factor r of butterfly jm at
+// (r-1)*ns + jm of its stage, so that lanes along jm read consecutive entries.
+template <typename T>
+std::vector<cpx<T>> stage_twiddles_gen(const std::vector<int>& radices, std::vector<int>* offs) {
+    std::vector<cpx<T>> tw;
+    int64_t ns = 1;
+    for (int R : radices) {
+        offs->push_back((int)tw.size());
+        if (ns > 1)
+            for (int r = 1; r < R; r++)
+                for (int64_t jm = 0; jm < ns; jm++) tw.push_back(expm<T>(jm * r, ns * R));
         ns *= R;
     }
     if (tw.empty()) tw.push_back(cpx<T>{T(1), T(0)});
@@ -284,9 +333,24 @@ std::unique_ptr<Fft1D<T>> make_fft1d(int64_t n) {
     bool tpl = tpl_radices(n, r);
     if (tpl || (n <= gen_max<T>() && factor_radices(n, r))) {
         p->kind = tpl ? K_TPL : K_GEN;
+        if (!tpl) {
+            r = gen_radices(n);
+            std::vector<int> offs;
+            upload(p->tw, stage_twiddles_gen<T>(r, &offs));
+            p->radices = r;
+            GenPlan& g = p->gp;
+            g.n = (int)n;
+            g.nst = (int)r.size();
+            int ns = 1;
+            for (size_t i = 0; i < r.size(); i++) {
+                const int m = (int)(n / r[i]);
+                g.st[i] = GenStage{r[i], m, ns, offs[i], 1.0f / (float)m, 1.0f / (float)ns};
+                ns *= r[i];
+            }
+            return p;
+        }
         p->radices = r;
-        std::vector<int> offs;
-        std::vector<cpx<T>> tab = stage_twiddles<T>(r, &offs);
+        std::vector<cpx<T>> tab = stage_twiddles<T>(r, nullptr);
         if (n == 4096) {
             // the 4096-point complex row kernels run radices 16,8,8,4; their
             // table follows the 16,16,16 one (see dispatch_tpl_n)
@@ -298,12 +362,6 @@ std::unique_ptr<Fft1D<T>> make_fft1d(int64_t n) {
             tab.insert(tab.end(), t2.begin(), t2.end());
         }
         upload(p->tw, tab);
-        p->gp.n = (int)n;
-        p->gp.nstages = (int)r.size();
-        for (size_t i = 0; i < r.size(); i++) {
-            p->gp.radix[i] = r[i];
-            p->gp.twoff[i] = offs[i];
-        }
         return p;
     }
     if (factor_radices(n, r)) {
@@ -543,14 +601,75 @@ bool dispatch_tpl(int64_t n, IO io, const cpx<T>* tw, hipStream_t st, bool mf = 
     return dispatch_tpl_n<T, DIR, COL>(n, io, tw, st);
 }
 
+// Launch shape of the runtime-radix kernel: W lines and NT threads per
+// workgroup.  eb: bytes of one element of a line in memory.  The lines lie
+// where these were fastest (us for a forward and a backward pass):
+//   - columns of 128-B segments while two workgroups share a CU: 180^3 FP64
+//     200 at 64 or 128 B, 205 at 256 B; DCT 300x200x180 338 against 360;
+//   - fewer lines per workgroup only below 192 workgroups: 1080 x 1920 FP32
+//     58 with 240 workgroups of 8 columns, 62 with 480 of 4; 360 x 640 FP32
+//     33 against 31 the other way round;
+//   - rows of up to 2048 points per workgroup: 10000 x 1000 FP64 132 (1024
+//     points: 130, 4096: 142), DCT 300x200x180 338 (344, 397);
+//   - at least one thread per 8 points: 3000 x 2000 FP32 148 against 164 with
+//     one per 16; one per 4 only while the chip is not full (360 x 640 26.5
+//     against 28.6, but 3000 x 2000 180).  Hooks have O(n) work of their own:
+//     up to one per 2 points there (DST 1000 x 1000 FP64 53 against 72).
+struct GenShape {
+    int W, NT;
+    size_t shm;
+};
+template <typename T>
+GenShape gen_shape(GenPlan& g, int64_t nlines, bool col, int eb, bool hooks) {
+    const int n = g.n;
+    auto pitch_of = [&](int W) {
+        // lines fall into disjoint bank groups (as LdsGeom)
+        const int p = n + (n >> 5) + 1;
+        const int off = 16 / W > 0 ? 16 / W : 1;
+        return W == 1 ? p : p + (off - p % 32 + 64) % 32;
+    };
+    auto threads = [&](int W) {
+        int nt = 64;
+        for (int s = 0; s < g.nst; s++) {
+            const int per = gen_butterflies(g.st[s].radix);
+            nt = std::max(nt, (g.st[s].m * W + per - 1) / per);
+        }
+        if (!hooks) nt = std::max(nt, std::min(1024, n * W / 8));
+        return (nt + 63) / 64 * 64;
+    };
+    auto bytes = [&](int W) { return 2 * (size_t)W * pitch_of(W) * sizeof(T); };
+    auto fits = [&](int W, size_t lds) { return W <= 64 && threads(W) <= 1024 && bytes(W) <= lds; };
+    auto groups = [&](int W) { return (nlines + W - 1) / W; };
+    int W = 1;
+    if (col) {
+        // 128-B row segments while two workgroups share a CU's LDS, else 64-B
+        // ones; short lines fill a wave; narrower where the chip would idle
+        while (2 * W * eb <= 128 && fits(2 * W, 80 * 1024)) W *= 2;
+        while (2 * W * eb <= 64 && fits(2 * W, 160 * 1024)) W *= 2;
+        while (W < 16 && W * n < 1024 && fits(2 * W, 80 * 1024)) W *= 2;
+        while (W > 1 && W * eb > 32 && groups(W) < 192) W /= 2;
+    } else {
+        while (2 * W * n <= 2048 && fits(2 * W, 80 * 1024)) W *= 2;
+        while (W > 1 && groups(W) < 512) W /= 2;
+    }
+    int nt = threads(W);
+    // few lines: more threads per line hide more of each stage's latency
+    const int most = std::min(1024, n * W / (hooks ? 2 : 4));
+    while (2 * nt <= most && groups(W) * nt < (int64_t(1) << 18)) nt *= 2;
+    if (!fits(W, 160 * 1024)) throw JtError(ST_UNSUPPORTED, "internal: length beyond the runtime-radix kernel");
+    g.W = W;
+    g.lgW = 0;
+    while ((1 << g.lgW) < W) g.lgW++;
+    g.col = col ? 1 : 0;
+    g.pitch = pitch_of(W);
+    return GenShape{W, nt, bytes(W)};
+}
+
 template <typename T, int DIR, class IO>
-void go_gen(const Fft1D<T>& p, IO io, hipStream_t st) {
+void go_gen(const Fft1D<T>& p, IO io, bool col, hipStream_t st) {
     if (io.nlines <= 0) return;
-    int n = (int)p.n;
-    int np = n + (n >> 5) + 1;
-    size_t shm = 4 * (size_t)np * sizeof(T);
-    int nt = n / 4;
-    nt = nt < 64 ? 64 : (nt > 256 ? 256 : ((nt + 63) / 64) * 64);
+    GenPlan g = p.gp;
+    const GenShape sh = gen_shape<T>(g, io.nlines, col, (int)(io_real_lines<IO>::value ? sizeof(T) : sizeof(cpx<T>)), IO::pre_lds || IO::post_lds);
     // the LDS limit is raised once per instantiation and device
     static std::atomic<uint64_t> attr_devs{0};
     int dev = 0;
@@ -561,13 +680,13 @@ void go_gen(const Fft1D<T>& p, IO io, hipStream_t st) {
                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         attr_devs.fetch_or(bit);
     }
-    int64_t lines = io.nlines;
-    JT_PROF(st, std::string("generic<") + (sizeof(T) == 8 ? "f64" : "f32") + ",N=" + std::to_string(n) +
-                    ",lines=" + std::to_string(lines) + "," + IO::tag() + io.desc() + ">");
-    unsigned gx = (unsigned)(lines < 65535 ? lines : 65535);
-    unsigned gy = (unsigned)((lines + gx - 1) / gx);
-    hipLaunchKernelGGL((generic_kernel<T, DIR, IO>), dim3(gx, gy), dim3(nt), shm, st, io,
-                       p.tw.template as<cpx<T>>(), p.gp);
+    JT_PROF(st, std::string("generic<") + (sizeof(T) == 8 ? "f64" : "f32") + ",N=" + std::to_string(g.n) +
+                    (col ? ",col" : ",row") + ",W=" + std::to_string(sh.W) + ",NT=" + std::to_string(sh.NT) +
+                    ",lines=" + std::to_string(io.nlines) + "," + IO::tag() + io.desc() + ">");
+    const int64_t groups = (io.nlines + sh.W - 1) / sh.W;
+    const int64_t gx = std::min<int64_t>(groups, int64_t(1) << 20);
+    hipLaunchKernelGGL((generic_kernel<T, DIR, IO>), dim3((unsigned)gx, (unsigned)((groups + gx - 1) / gx)),
+                       dim3(sh.NT), sh.shm, st, io, p.tw.template as<cpx<T>>(), g);
     JT_HIP(hipGetLastError());
 }
 
@@ -579,9 +698,8 @@ void run_single(const Fft1D<T>& p, IO io, hipStream_t st) {
                                       p.tw_mf.template as<cpx<T>>()))
             return;
     }
-    if (p.kind == K_GEN || p.kind == K_TPL) {
-        // generic kernel needs a radix plan
-        go_gen<T, DIR>(p, io, st);
+    if (p.kind == K_GEN) {
+        go_gen<T, DIR>(p, io, COL, st);
         return;
     }
     throw JtError(ST_UNSUPPORTED, "run_single on a multi-pass plan");
@@ -703,12 +821,17 @@ void c2c_contig(const Fft1D<T>& p, const cpx<T>* in, cpx<T>* out, int64_t lines,
     }
     if (p.kind == K_FOUR) {
         if (!p.p1->single()) throw JtError(ST_UNSUPPORTED, "four-step column plan must be single-kernel");
+        const bool two = p.p2->single();
         IOFourA<T, DIR> a{in, ws, p.hi.template as<cpx<T>>(), p.lo.template as<cpx<T>>(), lines * p.n2,
-                          p.n, p.n1, p.n2, true};
+                          p.n, p.n1, p.n2, two ? p.n1 : 1, two ? 1 : p.n2, true};
         run_single<T, DIR, true>(*p.p1, a, st);
-        if (p.p2->single()) {
-            IOFourB<T> b{ws, out, lines * p.n1, p.n, p.n1, p.n2, scale, false};
-            run_single<T, DIR, false>(*p.p2, b, st);
+        if (two) {
+            // pass A left the transpose: the n2-point rows are columns of an
+            // n2 x n1 matrix, and their results go to the same places of
+            // `out`, so both passes read and write whole segments.  (Rows
+            // with a transposing store of single 16-byte points: FP64
+            // 3072 x 4096 points 203 us for pass B, as columns 113.)
+            c2c_mapped<T, DIR>(*p.p2, ws, out, LineMap{lines * p.n1, p.n1, 1, p.n, p.n1}, scale, st);
             return;
         }
         // long rows: FFT them in place in the workspace, then transpose
@@ -742,5 +865,15 @@ void c2c_contig(const Fft1D<T>& p, const cpx<T>* in, cpx<T>* out, int64_t lines,
     }
     JT_HIP(hipGetLastError());
 }
+
+// Instantiated in jt_c2c_*.hip, one precision and direction each, so that the
+// kernels compile in parallel.
+#define JT_C2C_INST(X, T, D)                                                                                     \
+    X template void c2c_mapped<T, D>(const Fft1D<T>&, const cpx<T>*, cpx<T>*, LineMap, T, hipStream_t, int);       \
+    X template void c2c_contig<T, D>(const Fft1D<T>&, const cpx<T>*, cpx<T>*, int64_t, T, cpx<T>*, hipStream_t);
+JT_C2C_INST(extern, float, -1)
+JT_C2C_INST(extern, float, 1)
+JT_C2C_INST(extern, double, -1)
+JT_C2C_INST(extern, double, 1)
 
 }  // namespace jt

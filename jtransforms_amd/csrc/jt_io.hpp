@@ -13,7 +13,15 @@ __device__ __forceinline__ int lpos(int k) { return k + (k >> 5); }
 // element k of a line sits es further per step.
 struct LineMap {
     int64_t nlines, n0, s0, s1, es;
-    __device__ __forceinline__ int64_t base(int64_t l) const { return (l % n0) * s0 + (l / n0) * s1; }
+    __device__ __forceinline__ int64_t base(int64_t l) const {
+        // (a 64-bit division by a run-time value takes over a hundred instructions)
+        if (nlines <= n0) return l * s0;
+        if (((uint64_t)nlines | (uint64_t)n0) >> 32 == 0) {
+            const uint32_t q = (uint32_t)l / (uint32_t)n0;
+            return (int64_t)((uint32_t)l - q * (uint32_t)n0) * s0 + (int64_t)q * s1;
+        }
+        return (l % n0) * s0 + (l / n0) * s1;
+    }
 };
 
 // Non-temporal (streaming) complex loads and stores: they skip the caches'
@@ -40,7 +48,7 @@ enum { NT_LOAD = 1, NT_STORE = 2 };
 // kernels registers and load batching.
 template <typename T, int NT = 0>
 struct IOStrided {
-    static constexpr bool pre_lds = false, post_lds = false;
+    static constexpr bool pre_lds = false, post_lds = false, store_loads = false;
     static constexpr int streaming = NT;
     static const char* tag() { return NT == 0 ? "c2c" : "c2c,nt"; }
     std::string desc() const { return ",es=" + std::to_string(m.es); }
@@ -51,18 +59,20 @@ struct IOStrided {
     T scale;
     bool xcd;
     __device__ __forceinline__ int64_t base(int64_t l) const { return m.base(l); }
-    __device__ __forceinline__ cpx<T> load(int64_t b, int k) const {
-        if constexpr ((NT & NT_LOAD) != 0) return ld_nt(in + b + k * m.es);
-        else return in[b + k * m.es];
+    __device__ __forceinline__ cpx<T> load(int64_t b, int k, int rm) const {
+        const cpx<T>* p = in + (b + k * m.es) + rm * m.es;
+        if constexpr ((NT & NT_LOAD) != 0) return ld_nt(p);
+        else return *p;
     }
     // one part (0 real, 1 imaginary) of element k
     __device__ __forceinline__ T loadf(int64_t b, int k, int part) const {
         return reinterpret_cast<const T*>(in + b + k * m.es)[part];
     }
-    __device__ __forceinline__ void store(int64_t b, int k, cpx<T> v) const {
+    __device__ __forceinline__ void store(int64_t b, int k, int rm, cpx<T> v) const {
         const cpx<T> o{v.x * scale, v.y * scale};
-        if constexpr ((NT & NT_STORE) != 0) st_nt(out + b + k * m.es, o);
-        else out[b + k * m.es] = o;
+        cpx<T>* p = out + (b + k * m.es) + rm * m.es;
+        if constexpr ((NT & NT_STORE) != 0) st_nt(p, o);
+        else *p = o;
     }
     template <int CN, int CTL>
     __device__ void pre(int64_t, int64_t, T*, T*, int, int) const {}
@@ -112,55 +122,37 @@ __device__ __forceinline__ cpx<T> tw2(const cpx<T>* __restrict__ hi, const cpx<T
 
 // Four-step pass A: transform length n = n1*n2 viewed as an n1 x n2 row-major
 // matrix.  Line (b, j2) is column j2 of batch b (n1 points at stride n2); the
-// result is multiplied by exp(DIR 2 pi i j2 k1 / n) and written to the same
-// position of `out`.
+// result is multiplied by exp(DIR 2 pi i j2 k1 / n) and point k1 of column j2
+// written to b*n + j2*oj + k1*ok: transposed (oj = n1, ok = 1) when the rows
+// follow as columns of that n2 x n1 matrix, or in place (oj = 1, ok = n2).
 template <typename T, int DIR>
 struct IOFourA {
-    static constexpr bool pre_lds = false, post_lds = false;
+    static constexpr bool pre_lds = false, post_lds = false, store_loads = true;
     static const char* tag() { return "fourA"; }
     std::string desc() const { return ",n1=" + std::to_string(n1) + ",n2=" + std::to_string(n2); }
     const cpx<T>* in;
     cpx<T>* out;
     const cpx<T>* hi;
     const cpx<T>* lo;
-    int64_t nlines, n, n1, n2;
+    int64_t nlines, n, n1, n2, oj, ok;
     bool xcd;
-    __device__ __forceinline__ int64_t base(int64_t l) const { return (l / n2) * n + (l % n2); }
-    __device__ __forceinline__ cpx<T> load(int64_t b, int k) const { return in[b + (int64_t)k * n2]; }
-    __device__ __forceinline__ void store(int64_t b, int k, cpx<T> v) const {
-        int64_t j2 = b % n;  // column index inside the batch entry
-        int64_t e = (j2 * (int64_t)k) % n;
-        out[b + (int64_t)k * n2] = cmul(v, tw2<DIR>(hi, lo, e));
+    struct At {
+        int64_t i, o, j2;
+    };
+    __device__ __forceinline__ At base(int64_t l) const {
+        if (nlines == n2) return At{l, l * oj, l};  // one transform
+        const int64_t b = l / n2, j2 = l - b * n2;
+        return At{b * n + j2, b * n + j2 * oj, j2};
+    }
+    __device__ __forceinline__ cpx<T> load(At a, int k, int rm) const { return in[(a.i + k * n2) + rm * n2]; }
+    __device__ __forceinline__ void store(At a, int k, int rm, cpx<T> v) const {
+        const int64_t e = a.j2 * k + a.j2 * rm;  // j2 k1 < n2 n1: no reduction needed
+        out[(a.o + k * ok) + rm * ok] = cmul(v, tw2<DIR>(hi, lo, e));
     }
     template <int CN, int CTL>
-    __device__ void pre(int64_t, int64_t, T*, T*, int, int) const {}
+    __device__ void pre(int64_t, At, T*, T*, int, int) const {}
     template <int CN, int CTL>
-    __device__ void post(int64_t, int64_t, const T*, const T*, int, int) const {}
-};
-
-// Four-step pass B: line (b, k1) is row k1 (n2 contiguous points); output
-// point k2 is X[k1 + n1*k2], written with stride n1.
-template <typename T>
-struct IOFourB {
-    static constexpr bool pre_lds = false, post_lds = false;
-    static const char* tag() { return "fourB"; }
-    std::string desc() const { return ",n1=" + std::to_string(n1) + ",n2=" + std::to_string(n2); }
-    const cpx<T>* in;
-    cpx<T>* out;
-    int64_t nlines, n, n1, n2;
-    T scale;
-    bool xcd;
-    // base encodes (b, k1) as b*n + k1*n2 (the input row start)
-    __device__ __forceinline__ int64_t base(int64_t l) const { return (l / n1) * n + (l % n1) * n2; }
-    __device__ __forceinline__ cpx<T> load(int64_t b, int k) const { return in[b + k]; }
-    __device__ __forceinline__ void store(int64_t b, int k, cpx<T> v) const {
-        int64_t bb = b / n, k1 = (b % n) / n2;
-        out[bb * n + k1 + (int64_t)k * n1] = cpx<T>{v.x * scale, v.y * scale};
-    }
-    template <int CN, int CTL>
-    __device__ void pre(int64_t, int64_t, T*, T*, int, int) const {}
-    template <int CN, int CTL>
-    __device__ void post(int64_t, int64_t, const T*, const T*, int, int) const {}
+    __device__ void post(int64_t, At, const T*, const T*, int, int) const {}
 };
 
 // realForward post pass (reference: CommonUtils.rftfsub :5750-5776 and the
@@ -171,7 +163,7 @@ struct IOFourB {
 // w = exp(-2 pi i/2N).  rtw[k] = w^k for k in [0, N/2].
 template <typename T>
 struct IOR2C {
-    static constexpr bool pre_lds = false, post_lds = true;
+    static constexpr bool pre_lds = false, post_lds = true, store_loads = false;
     static const char* tag() { return "r2c"; }
     std::string desc() const { return ",es=" + std::to_string(m.es); }
     const cpx<T>* in;  // reals viewed as complex pairs
@@ -183,8 +175,8 @@ struct IOR2C {
     T scale;
     bool xcd;
     __device__ __forceinline__ int64_t base(int64_t l) const { return m.base(l); }
-    __device__ __forceinline__ cpx<T> load(int64_t b, int k) const { return in[b + k]; }
-    __device__ void store(int64_t, int, cpx<T>) const {}
+    __device__ __forceinline__ cpx<T> load(int64_t b, int k, int rm) const { return in[b + k + rm]; }
+    __device__ void store(int64_t, int, int, cpx<T>) const {}
     template <int CN, int CTL>
     __device__ void pre(int64_t, int64_t, T*, T*, int, int) const {}
     template <int CN, int CTL>
@@ -199,7 +191,7 @@ struct IOR2C {
         const int n = CN > 0 ? CN : N;
         const int step = CTL > 0 ? CTL : nt;
         // k = 1 .. n/2, with compile-time trip counts when CN, CTL are known
-        constexpr int ITER = (CN > 0 && CTL > 0) ? (CN / 2 + CTL - 1) / CTL : 1;
+        constexpr int ITER = (CN > 0 && CTL > 0) ? (CN / 2 + CTL - 1) / CTL : 4;
         for (int k0 = 1 + t; k0 <= n / 2; k0 += ITER * step) {
 #pragma unroll
             for (int i = 0; i < ITER; i++) {
@@ -227,7 +219,7 @@ struct IOR2C {
 // is sum-normalised (x_{2m} + i x_{2m+1}) * 2N, stored times `scale`.
 template <typename T>
 struct IOC2R {
-    static constexpr bool pre_lds = true, post_lds = false;
+    static constexpr bool pre_lds = true, post_lds = false, store_loads = false;
     static const char* tag() { return "c2r"; }
     std::string desc() const { return ",es=" + std::to_string(m.es); }
     const T* in;     // packed reals
@@ -239,9 +231,9 @@ struct IOC2R {
     T scale;
     bool xcd;
     __device__ __forceinline__ int64_t base(int64_t l) const { return m.base(l); }
-    __device__ cpx<T> load(int64_t, int) const { return cpx<T>{T(0), T(0)}; }
-    __device__ __forceinline__ void store(int64_t b, int k, cpx<T> v) const {
-        out[b + k] = cpx<T>{v.x * scale, v.y * scale};
+    __device__ cpx<T> load(int64_t, int, int) const { return cpx<T>{T(0), T(0)}; }
+    __device__ __forceinline__ void store(int64_t b, int k, int rm, cpx<T> v) const {
+        out[b + k + rm] = cpx<T>{v.x * scale, v.y * scale};
     }
     // Z_k and Z_{N-k} from X_k, X_{N-k} (k in (0, N/2]); Z_0 from X_0, X_N
     __device__ __forceinline__ void c2r_pair(int k, cpx<T> Xk, cpx<T> Xn, T* re, T* im) const {
@@ -287,8 +279,24 @@ struct IOC2R {
                 if (k <= CN / 2) c2r_pair(k, xk[q], xn[q], re, im);
             }
         } else {
-            for (int k = 1 + t; k <= N / 2; k += nt)
-                c2r_pair(k, cpx<T>{a[2 * k], a[2 * k + 1]}, cpx<T>{a[2 * (N - k)], a[2 * (N - k) + 1]}, re, im);
+            // a few points at a time, their loads issued together
+            constexpr int IT = 4;
+            for (int k0 = 1 + t; k0 <= N / 2; k0 += IT * nt) {
+                cpx<T> xk[IT], xn[IT];
+#pragma unroll
+                for (int q = 0; q < IT; q++) {
+                    const int k = k0 + q * nt;
+                    if (k <= N / 2) {
+                        xk[q] = cpx<T>{a[2 * k], a[2 * k + 1]};
+                        xn[q] = cpx<T>{a[2 * (N - k)], a[2 * (N - k) + 1]};
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < IT; q++) {
+                    const int k = k0 + q * nt;
+                    if (k <= N / 2) c2r_pair(k, xk[q], xn[q], re, im);
+                }
+            }
         }
     }
     template <int CN, int CTL>

@@ -127,7 +127,7 @@ __global__ void __launch_bounds__(N / 16 * W) mfma_stockham_kernel(IO io, const 
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             const int k = et + TL * i;
-            cpx<float> v = io.load(ebase, k);
+            cpx<float> v = io.load(ebase, k, 0);
             lre[ew * G::pitch + lds_pos<N>(k)] = v.x;
             lim[ew * G::pitch + lds_pos<N>(k)] = v.y;
         }
@@ -241,7 +241,7 @@ __global__ void __launch_bounds__(N / 16 * W) mfma_stockham_kernel(IO io, const 
             }
             if (eact) {
 #pragma unroll
-                for (int i = 0; i < 16; i++) eio.store(ebase, et + TL * i, v[i]);
+                for (int i = 0; i < 16; i++) eio.store(ebase, et + TL * i, 0, v[i]);
             }
         } else {
             constexpr int NSL = N / R;
@@ -253,7 +253,7 @@ __global__ void __launch_bounds__(N / 16 * W) mfma_stockham_kernel(IO io, const 
 #pragma unroll
                 for (int q = 0; q < 16 / R; q++)
 #pragma unroll
-                    for (int r = 0; r < R; r++) eio.store(ebase, et + TL * (q + r * (16 / R)), v[q * R + r]);
+                    for (int r = 0; r < R; r++) eio.store(ebase, et + TL * (q + r * (16 / R)), 0, v[q * R + r]);
             }
         }
     }

@@ -52,7 +52,7 @@ inline R2RScale dct3_scale(int64_t n, bool scale) {
 // ---------------------------------------------------------------------------
 template <typename T, int KIND, bool FWD>
 struct IOR2R {
-    static constexpr bool pre_lds = true, post_lds = true;
+    static constexpr bool pre_lds = true, post_lds = true, store_loads = false;
     // lines of reals: a column group's row segment is W * sizeof(T) bytes
     static constexpr bool real_lines = true;
     static const char* tag() {
@@ -68,8 +68,8 @@ struct IOR2R {
     T f0, g;
     bool xcd;
     __device__ __forceinline__ int64_t base(int64_t l) const { return m.base(l); }
-    __device__ cpx<T> load(int64_t, int) const { return cpx<T>{T(0), T(0)}; }
-    __device__ void store(int64_t, int, cpx<T>) const {}
+    __device__ cpx<T> load(int64_t, int, int) const { return cpx<T>{T(0), T(0)}; }
+    __device__ void store(int64_t, int, int, cpx<T>) const {}
 
     __device__ __forceinline__ T rd(int64_t b, int k) const { return data[b + (int64_t)k * m.es]; }
     __device__ __forceinline__ void wr(int64_t b, int k, T v) const { data[b + (int64_t)k * m.es] = v; }
@@ -129,7 +129,17 @@ struct IOR2R {
 #pragma unroll
                 for (int q2 = 0; q2 < IT; q2++) put_fwd(t + q2 * CTL, vals[q2], re, im);
             } else {
-                for (int i = t; i < n; i += nt) put_fwd(i, fwd_in(b, i), re, im);
+                // a few points at a time, their loads issued together
+                constexpr int IT = 8;
+                for (int i0 = t; i0 < n; i0 += IT * nt) {
+                    T vals[IT];
+#pragma unroll
+                    for (int q2 = 0; q2 < IT; q2++)
+                        if (i0 + q2 * nt < n) vals[q2] = fwd_in(b, i0 + q2 * nt);
+#pragma unroll
+                    for (int q2 = 0; q2 < IT; q2++)
+                        if (i0 + q2 * nt < n) put_fwd(i0 + q2 * nt, vals[q2], re, im);
+                }
             }
         } else {
             // DCT-III / DST-III: V_k = conj(q_k)(a'_k - i a'_{n-k}), then the
@@ -159,8 +169,25 @@ struct IOR2R {
                     if (k <= CN / 2) inv_pair(k, a0[q2], a1[q2], a2[q2], a3[q2], re, im);
                 }
             } else {
-                for (int k = 1 + t; k <= N / 2; k += nt)
-                    inv_pair(k, ain(b, k), ain(b, n - k), ain(b, N - k), ain(b, N + k), re, im);
+                constexpr int IT = 2;
+                for (int k0 = 1 + t; k0 <= N / 2; k0 += IT * nt) {
+                    T a0[IT], a1[IT], a2[IT], a3[IT];
+#pragma unroll
+                    for (int q2 = 0; q2 < IT; q2++) {
+                        const int k = k0 + q2 * nt;
+                        if (k <= N / 2) {
+                            a0[q2] = ain(b, k);
+                            a1[q2] = ain(b, n - k);
+                            a2[q2] = ain(b, N - k);
+                            a3[q2] = ain(b, N + k);
+                        }
+                    }
+#pragma unroll
+                    for (int q2 = 0; q2 < IT; q2++) {
+                        const int k = k0 + q2 * nt;
+                        if (k <= N / 2) inv_pair(k, a0[q2], a1[q2], a2[q2], a3[q2], re, im);
+                    }
+                }
             }
         }
     }
@@ -469,5 +496,12 @@ void run_r2r_nd(int family, int nd, const int64_t* d, const std::shared_ptr<R2R1
         JT_HIP(hipGetLastError());
     }
 }
+
+// Instantiated in jt_r2r_f64.hip and jt_r2r_f32.hip.
+#define JT_R2R_INST(X, T)                                                                                        \
+    X template void run_r2r_nd<T>(int, int, const int64_t*, const std::shared_ptr<R2R1D<T>>*, T*, bool, bool,      \
+                                  cpx<T>*, hipStream_t);
+JT_R2R_INST(extern, float)
+JT_R2R_INST(extern, double)
 
 }  // namespace jt

@@ -1,0 +1,6 @@
+// FP32 DCT, DST and DHT.
+#include "jt_r2r.hpp"
+
+namespace jt {
+JT_R2R_INST(, float)
+}  // namespace jt

@@ -19,6 +19,7 @@
 #include <type_traits>
 
 #include "jt_dft.hpp"
+#include "jt_generic.hpp"
 
 namespace jt {
 
@@ -194,17 +195,6 @@ struct FirstRadix {
     static constexpr int value = R0;
 };
 
-// Map workgroup id to line group so that consecutive groups (adjacent in
-// memory) land on the same XCD (workgroups are dispatched round-robin over
-// the 8 XCDs); keeps partial cache lines of neighbouring groups in one L2.
-__device__ __forceinline__ int64_t xcd_group(int64_t bid, int64_t ngroups) {
-    const int64_t nx = 8;
-    int64_t per = ngroups / nx;
-    int64_t full = per * nx;
-    if (bid >= full) return bid;
-    return (bid % nx) * per + bid / nx;
-}
-
 // IO policies that finish line 0 in place declare `static constexpr int
 // line0_hook` (> 0: after the line's stores, < 0: before its loads) and
 // `__device__ void line0(int tid, int nthreads)`.
@@ -217,9 +207,11 @@ struct io_line0_hook<IO, std::void_t<decltype(IO::line0_hook)>>
 // ----------------------------------------------------------------------------
 // The kernel.  IO supplies:
 //   int64_t nlines;  bool xcd;
-//   __device__ int64_t base(int64_t line)               element-0 offset
-//   __device__ cpx<T> load(int64_t base, int k)          element k of the line
-//   __device__ void store(int64_t base, int k, cpx<T>)   element k of the result
+//   __device__ At base(int64_t line)                     where the line is: its
+//              element-0 offset, or a struct of the policy's own
+//   __device__ cpx<T> load(At base, int k, int rm)        element k + rm of the line
+//   __device__ void store(At base, int k, int rm, cpx<T>) element k + rm of the result
+//              (rm: a part of the index that is uniform over the workgroup)
 //   static constexpr bool pre_lds, post_lds;
 //   pre_lds : __device__ void pre(int64_t line, int64_t base, T* re, T* im, int t)
 //             fills the line's LDS slots (re/im arrays, index lds_pos(k)) with
@@ -247,7 +239,7 @@ __global__ void __launch_bounds__(TL* W) stockham_kernel(IO io, const cpx<T>* __
     const int64_t g = io.xcd ? xcd_group(blockIdx.x, ngroups) : (int64_t)blockIdx.x;
     const int64_t line = g * W + w;
     const bool active = line < io.nlines;
-    const int64_t base = active ? io.base(line) : 0;
+    const auto base = io.base(active ? line : 0);
 
     if constexpr (io_line0_hook<IO>::value < 0) {
         // the workgroup that holds line 0 rewrites it before anyone loads it
@@ -271,7 +263,7 @@ __global__ void __launch_bounds__(TL* W) stockham_kernel(IO io, const cpx<T>* __
 #pragma unroll
             for (int r = 0; r < R0; r++) {
                 int k = t + TL * (q + r * (E / R0));
-                v[q * R0 + r] = active ? io.load(base, k) : cpx<T>{T(0), T(0)};
+                v[q * R0 + r] = active ? io.load(base, k, 0) : cpx<T>{T(0), T(0)};
             }
     }
 
@@ -287,7 +279,7 @@ __global__ void __launch_bounds__(TL* W) stockham_kernel(IO io, const cpx<T>* __
 #pragma unroll
                 for (int r = 0; r < RL; r++) {
                     int k = t + TL * (q + r * (E / RL));
-                    io.store(base, k, v[q * RL + r]);
+                    io.store(base, k, 0, v[q * RL + r]);
                 }
         }
     }

@@ -1,0 +1,67 @@
+"""The runtime-radix kernel (lengths without a compile-time kernel) at the
+edges of its shapes: every radix alone and as the first, an inner and the last
+stage, the longest lengths, one line, and line counts that leave the last
+workgroup partly filled, over rows (batches) and columns (first axis of a 2D
+transform).  Tolerances as in test_gpu_fft: FP64 rel-l2 <= 1e-13 * log2(N),
+FP32 <= 2e-7 * log2(N) + 1e-6, against the FP64 oracle."""
+import math
+
+import numpy as np
+import pytest
+
+import jtransforms_amd as jt
+
+pytestmark = pytest.mark.gpu
+
+DT = {"f64": np.float64, "f32": np.float32}
+FFT2 = {"f64": jt.DoubleFFT_2D, "f32": jt.FloatFFT_2D}
+
+# one stage; two; three and more (2197 = 13^3, 3125 = 5^5, 3993 = 3 * 11^3); the limits
+LENGTHS = [2, 3, 5, 6, 7, 9, 10, 11, 12, 13, 14, 15, 18, 33, 91, 98, 132, 143, 180, 225, 1000, 1331, 2197, 3125, 3993,
+           4095]
+LENGTHS_F32 = [5000, 6655, 7203, 7290, 8192]
+
+
+def tol(n, prec):
+    lg = max(1.0, math.log2(max(n, 2)))
+    return 1e-13 * lg if prec == "f64" else 2e-7 * lg + 1e-6
+
+
+def rel(a, b):
+    a = np.asarray(a, np.float64).ravel()
+    b = np.asarray(b, np.float64).ravel()
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+CASES = [(n, p) for p in ("f64", "f32") for n in LENGTHS] + [(n, "f32") for n in LENGTHS_F32]
+
+
+@pytest.mark.parametrize("n,prec", CASES)
+def test_rows(orc, n, prec):
+    for lines in (1, 3, 65, 1030):
+        if n * lines > 1 << 20:
+            continue
+        x = orc.jrandom_doubles(n + lines, 2 * n * lines).astype(DT[prec])
+        p = jt.FFTBatch1D(n, lines, precision=prec)
+        a = x.copy()
+        p.complexForward(a)
+        for b in {0, lines // 2, lines - 1}:
+            seg = slice(2 * n * b, 2 * n * (b + 1))
+            assert rel(a[seg], orc.complex_forward(n, x[seg].astype(np.float64))) <= tol(n, prec), (n, lines, b)
+        p.complexInverse(a, True)
+        assert rel(a, x) <= 2 * tol(n, prec), (n, lines)
+
+
+@pytest.mark.parametrize("n,prec", CASES)
+def test_columns(orc, n, prec):
+    for cols in (3, 17, 250):
+        if n * cols > 1 << 18:
+            continue
+        x = orc.jrandom_doubles(n + cols, 2 * n * cols).astype(DT[prec])
+        p = FFT2[prec](n, cols)
+        a = x.copy()
+        p.complexForward(a)
+        e = rel(a, orc.fftnd_complex([n, cols], x.astype(np.float64), -1))
+        assert e <= tol(n * cols, prec), (n, cols, e)
+        p.complexInverse(a, True)
+        assert rel(a, x) <= 2 * tol(n * cols, prec), (n, cols)
