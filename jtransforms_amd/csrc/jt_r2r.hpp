@@ -47,6 +47,11 @@ inline R2RScale dct3_scale(int64_t n, bool scale) {
 
 // ---------------------------------------------------------------------------
 // fused IO policy.  Real data: element k of line l at data[base(l) + k*es].
+// Bound: HBM, as long as a batch's loads are in flight together.  The inverse
+// hook used to select per load (a_n = 0, a'_0 = f0 a_0), which put a wait
+// behind every load, and to write one element at a time from LDS: the three
+// DCT-III passes of 512^3 FP64 took 727, 775 and 743 us (2.9 TB/s); without
+// the selections, four elements at a time, 495, 502 and 582 (3.7-4.3).
 // N = n/2 complex points per line.  q[k] = exp(-i pi k / 2n), k in [0, n];
 // rtw[k] = exp(-2 pi i k / n), k in [0, n/4 + 1].
 // ---------------------------------------------------------------------------
@@ -74,31 +79,56 @@ struct IOR2R {
     __device__ __forceinline__ T rd(int64_t b, int k) const { return data[b + (int64_t)k * m.es]; }
     __device__ __forceinline__ void wr(int64_t b, int k, T v) const { data[b + (int64_t)k * m.es] = v; }
 
-    // forward input x_j with the DST sign map
-    __device__ __forceinline__ T xin(int64_t b, int j) const {
-        T v = rd(b, j);
-        if (KIND == R2R_DST && (j & 1)) v = -v;
-        return v;
-    }
-    // inverse input a'_k (DST reads reversed), 0 for k == n
-    __device__ __forceinline__ T ain(int64_t b, int k) const {
-        if (k >= n) return T(0);
-        T v = KIND == R2R_DST ? rd(b, n - 1 - k) : rd(b, k);
-        return k == 0 ? v * f0 : v;
-    }
+    // inverse input a_k (DST reads reversed); a'_0 = f0 a_0 is the caller's
+    __device__ __forceinline__ T ain(int64_t b, int k) const { return rd(b, KIND == R2R_DST ? n - 1 - k : k); }
 
-    // forward: element i of the line -> its slot in the N complex inputs
-    __device__ __forceinline__ void put_fwd(int i, T v, T* re, T* im) const {
-        int j;
-        if constexpr (KIND == R2R_DHT) j = i;  // natural pairs z_m = x_2m + i x_2m+1
-        else j = (i & 1) ? n - 1 - (i >> 1) : (i >> 1);  // Makhoul: v_j = x_2j, v_{n-1-j} = x_2j+1
-        int mm = j >> 1;
-        if (j & 1) im[lpos(mm)] = v;
-        else re[lpos(mm)] = v;
+    // Four consecutive elements i, .., i+3 of the line at a time: contiguous
+    // lines hold them in two aligned pairs (n is even and the data
+    // pair-aligned).
+    __device__ __forceinline__ void rd4(int64_t b, int i, T* x) const {
+        if (m.es == 1) {
+            const cpx<T>* p = reinterpret_cast<const cpx<T>*>(data + b + i);
+            const cpx<T> lo = p[0], hi = p[1];
+            x[0] = lo.x; x[1] = lo.y; x[2] = hi.x; x[3] = hi.y;
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; u++) x[u] = rd(b, i + u);
+        }
     }
-    __device__ __forceinline__ T fwd_in(int64_t b, int i) const {
-        if constexpr (KIND == R2R_DHT) return rd(b, i);
-        else return xin(b, i);
+    __device__ __forceinline__ void wr4(int64_t b, int i, const T* x) const {
+        if (m.es == 1) {
+            cpx<T>* p = reinterpret_cast<cpx<T>*>(data + b + i);
+            p[0] = cpx<T>{x[0], x[1]};
+            p[1] = cpx<T>{x[2], x[3]};
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; u++) wr(b, i + u, x[u]);
+        }
+    }
+    // Makhoul's order v_j = x_2j, v_{n-1-j} = x_{2j+1} with z_m = v_2m + i
+    // v_2m+1: elements 4h, .., 4h+3 are Re z_h, Im z_{N-1-h}, Im z_h and
+    // Re z_{N-1-h} (h < N/2; for odd N, x_{n-2} and x_{n-1} are z_{(N-1)/2}).
+    // The DHT keeps the natural order.
+    __device__ __forceinline__ void put4(int h, const T* x, T* re, T* im) const {
+        if constexpr (KIND == R2R_DHT) {
+            re[lpos(2 * h)] = x[0];
+            im[lpos(2 * h)] = x[1];
+            re[lpos(2 * h + 1)] = x[2];
+            im[lpos(2 * h + 1)] = x[3];
+        } else {
+            constexpr T sg = KIND == R2R_DST ? T(-1) : T(1);
+            re[lpos(h)] = x[0];
+            im[lpos(N - 1 - h)] = sg * x[1];
+            im[lpos(h)] = x[2];
+            re[lpos(N - 1 - h)] = sg * x[3];
+        }
+    }
+    // the last pair of a line with odd N
+    __device__ __forceinline__ void put_last(int64_t b, T* re, T* im) const {
+        const int z = KIND == R2R_DHT ? N - 1 : (N - 1) / 2;
+        const T y = rd(b, n - 1);
+        re[lpos(z)] = rd(b, n - 2);
+        im[lpos(z)] = KIND == R2R_DST ? -y : y;
     }
     // inverse: Z_k, Z_{N-k} from a'_k, a'_{n-k}, a'_{N-k}, a'_{N+k}
     __device__ __forceinline__ void inv_pair(int k, T ak, T ank, T akk, T ankk, T* re, T* im) const {
@@ -120,73 +150,51 @@ struct IOR2R {
     template <int CN, int CTL>
     __device__ void pre(int64_t, int64_t b, T* re, T* im, int t, int nt) const {
         if constexpr (FWD || KIND == R2R_DHT) {
-            if constexpr (CN > 0) {
-                // 2N reals per line: issue every load before the LDS writes
-                constexpr int IT = (2 * CN) / CTL;
-                T vals[IT];
+            // all loads of a batch before its LDS writes (compile-time
+            // lengths: one batch)
+            constexpr int IT = CN > 0 ? (CN / 2 + CTL - 1) / CTL : 2;
+            const int half = (CN > 0 ? CN : N) / 2, step = CTL > 0 ? CTL : nt;
+            for (int h0 = t; h0 < half; h0 += IT * step) {
+                T x[IT][4];
 #pragma unroll
-                for (int q2 = 0; q2 < IT; q2++) vals[q2] = fwd_in(b, t + q2 * CTL);
+                for (int u = 0; u < IT; u++)
+                    if (h0 + u * step < half) rd4(b, 4 * (h0 + u * step), x[u]);
 #pragma unroll
-                for (int q2 = 0; q2 < IT; q2++) put_fwd(t + q2 * CTL, vals[q2], re, im);
-            } else {
-                // a few points at a time, their loads issued together
-                constexpr int IT = 8;
-                for (int i0 = t; i0 < n; i0 += IT * nt) {
-                    T vals[IT];
-#pragma unroll
-                    for (int q2 = 0; q2 < IT; q2++)
-                        if (i0 + q2 * nt < n) vals[q2] = fwd_in(b, i0 + q2 * nt);
-#pragma unroll
-                    for (int q2 = 0; q2 < IT; q2++)
-                        if (i0 + q2 * nt < n) put_fwd(i0 + q2 * nt, vals[q2], re, im);
-                }
+                for (int u = 0; u < IT; u++)
+                    if (h0 + u * step < half) put4(h0 + u * step, x[u], re, im);
+            }
+            if constexpr (CN == 0) {
+                if ((N & 1) && t == 0) put_last(b, re, im);
             }
         } else {
             // DCT-III / DST-III: V_k = conj(q_k)(a'_k - i a'_{n-k}), then the
             // real-inverse split into Z (N points)
             if (t == 0) {
-                T v0 = ain(b, 0);
+                T v0 = ain(b, 0) * f0;
                 T vN = T(1.41421356237309504880168872420970) * ain(b, N);
                 re[lpos(0)] = v0 + vN;
                 im[lpos(0)] = v0 - vN;
             }
-            if constexpr (CN > 0) {
-                constexpr int IT = (CN / 2 + CTL - 1) / CTL;
+            // all loads of a batch before its LDS writes (compile-time
+            // lengths: one batch)
+            constexpr int IT = CN > 0 ? (CN / 2 + CTL - 1) / CTL : 2;
+            const int nn = CN > 0 ? CN : N, step = CTL > 0 ? CTL : nt;
+            for (int k0 = 1 + t; k0 <= nn / 2; k0 += IT * step) {
                 T a0[IT], a1[IT], a2[IT], a3[IT];
 #pragma unroll
-                for (int q2 = 0; q2 < IT; q2++) {
-                    int k = 1 + t + q2 * CTL;
-                    if (k <= CN / 2) {
-                        a0[q2] = ain(b, k);
-                        a1[q2] = ain(b, n - k);
-                        a2[q2] = ain(b, N - k);
-                        a3[q2] = ain(b, N + k);
+                for (int u = 0; u < IT; u++) {
+                    const int k = k0 + u * step;
+                    if (k <= nn / 2) {
+                        a0[u] = ain(b, k);
+                        a1[u] = ain(b, 2 * nn - k);
+                        a2[u] = ain(b, nn - k);
+                        a3[u] = ain(b, nn + k);
                     }
                 }
 #pragma unroll
-                for (int q2 = 0; q2 < IT; q2++) {
-                    int k = 1 + t + q2 * CTL;
-                    if (k <= CN / 2) inv_pair(k, a0[q2], a1[q2], a2[q2], a3[q2], re, im);
-                }
-            } else {
-                constexpr int IT = 2;
-                for (int k0 = 1 + t; k0 <= N / 2; k0 += IT * nt) {
-                    T a0[IT], a1[IT], a2[IT], a3[IT];
-#pragma unroll
-                    for (int q2 = 0; q2 < IT; q2++) {
-                        const int k = k0 + q2 * nt;
-                        if (k <= N / 2) {
-                            a0[q2] = ain(b, k);
-                            a1[q2] = ain(b, n - k);
-                            a2[q2] = ain(b, N - k);
-                            a3[q2] = ain(b, N + k);
-                        }
-                    }
-#pragma unroll
-                    for (int q2 = 0; q2 < IT; q2++) {
-                        const int k = k0 + q2 * nt;
-                        if (k <= N / 2) inv_pair(k, a0[q2], a1[q2], a2[q2], a3[q2], re, im);
-                    }
+                for (int u = 0; u < IT; u++) {
+                    const int k = k0 + u * step;
+                    if (k <= nn / 2) inv_pair(k, a0[u], a1[u], a2[u], a3[u], re, im);
                 }
             }
         }
@@ -203,55 +211,91 @@ struct IOR2R {
     template <int CN, int CTL>
     __device__ void post(int64_t, int64_t b, const T* re, const T* im, int t, int nt) const {
         if constexpr (FWD || KIND == R2R_DHT) {
-            // real-FFT split V_k / V_{N-k} from Z, then the transform outputs
-            for (int k = t; k <= N / 2; k += nt) {
-                if (k == 0) {
-                    T zr = re[lpos(0)], zi = im[lpos(0)];
-                    T V0 = zr + zi, VN = zr - zi;
-                    if constexpr (KIND == R2R_DHT) {
-                        out_fwd(b, 0, V0);
-                        out_fwd(b, N, VN);
-                    } else {
-                        out_fwd(b, 0, V0);
-                        out_fwd(b, N, T(0.70710678118654752440084436210485) * VN);
+            // real-FFT split V_k / V_{N-k} from Z, then the transform
+            // outputs.  A wait for a load also waits for older stores, so a
+            // batch loads all its factors first and stores last.
+            if (t == 0) {
+                const T zr = re[lpos(0)], zi = im[lpos(0)];
+                out_fwd(b, 0, zr + zi);
+                out_fwd(b, CN > 0 ? CN : N, KIND == R2R_DHT ? zr - zi : T(0.70710678118654752440084436210485) * (zr - zi));
+            }
+            constexpr int IT = CN > 0 ? ((CN / 2 + CTL - 1) / CTL < 4 ? (CN / 2 + CTL - 1) / CTL : 4) : 2;
+            const int nn = CN > 0 ? CN : N, step = CTL > 0 ? CTL : nt;
+            for (int k0 = 1 + t; k0 <= nn / 2; k0 += IT * step) {
+                cpx<T> w[IT], qa[IT], qb[IT];
+                T y[IT][4];
+#pragma unroll
+                for (int u = 0; u < IT; u++) {
+                    const int k = k0 + u * step;
+                    if (k > nn / 2) continue;
+                    w[u] = rtw[k];
+                    if constexpr (KIND != R2R_DHT) {
+                        qa[u] = q[k];
+                        qb[u] = q[nn - k];
                     }
-                    continue;
                 }
-                int kk = N - k;
-                cpx<T> A = {re[lpos(k)], im[lpos(k)]};
-                cpx<T> B = {re[lpos(kk)], -im[lpos(kk)]};
-                cpx<T> fe = cadd(A, B), d = csub(A, B);
-                cpx<T> fo = {d.y, -d.x};
-                cpx<T> wf = cmul(rtw[k], fo);
-                cpx<T> Vk = {(fe.x + wf.x) * T(0.5), (fe.y + wf.y) * T(0.5)};
-                cpx<T> Vc = {(fe.x - wf.x) * T(0.5), -(fe.y - wf.y) * T(0.5)};  // V_{N-k}
-                if constexpr (KIND == R2R_DHT) {
-                    out_fwd(b, k, Vk.x - Vk.y);
-                    out_fwd(b, n - k, Vk.x + Vk.y);
-                    if (kk != k) {
-                        out_fwd(b, kk, Vc.x - Vc.y);
-                        out_fwd(b, N + k, Vc.x + Vc.y);
+#pragma unroll
+                for (int u = 0; u < IT; u++) {
+                    const int k = k0 + u * step;
+                    if (k > nn / 2) continue;
+                    const int kk = nn - k;
+                    cpx<T> A = {re[lpos(k)], im[lpos(k)]};
+                    cpx<T> B = {re[lpos(kk)], -im[lpos(kk)]};
+                    cpx<T> fe = cadd(A, B), d = csub(A, B);
+                    cpx<T> fo = {d.y, -d.x};
+                    cpx<T> wf = cmul(w[u], fo);
+                    cpx<T> Vk = {(fe.x + wf.x) * T(0.5), (fe.y + wf.y) * T(0.5)};
+                    cpx<T> Vc = {(fe.x - wf.x) * T(0.5), -(fe.y - wf.y) * T(0.5)};  // V_{N-k}
+                    if constexpr (KIND == R2R_DHT) {
+                        y[u][0] = Vk.x - Vk.y;
+                        y[u][1] = Vk.x + Vk.y;
+                        y[u][2] = Vc.x - Vc.y;
+                        y[u][3] = Vc.x + Vc.y;
+                    } else {
+                        cpx<T> a = cmul(qa[u], Vk), c = cmul(qb[u], Vc);
+                        y[u][0] = a.x;
+                        y[u][1] = -a.y;
+                        y[u][2] = c.x;
+                        y[u][3] = -c.y;
                     }
-                } else {
-                    cpx<T> u = cmul(q[k], Vk);
-                    out_fwd(b, k, u.x);
-                    out_fwd(b, n - k, -u.y);
-                    if (kk != k) {
-                        cpx<T> uc = cmul(q[kk], Vc);
-                        out_fwd(b, kk, uc.x);
-                        out_fwd(b, N + k, -uc.y);
+                }
+#pragma unroll
+                for (int u = 0; u < IT; u++) {
+                    const int k = k0 + u * step;
+                    if (k > nn / 2) continue;
+                    out_fwd(b, k, y[u][0]);
+                    out_fwd(b, 2 * nn - k, y[u][1]);
+                    if (nn - k != k) {
+                        out_fwd(b, nn - k, y[u][2]);
+                        out_fwd(b, nn + k, y[u][3]);
                     }
                 }
             }
         } else {
             // inverse: LDS holds n * (v_2m + i v_2m+1); x_2j = v_j, x_2j+1 = v_{n-1-j}
-            for (int i = t; i < n; i += nt) {
-                int j = (i & 1) ? n - 1 - (i >> 1) : (i >> 1);
-                int mm = j >> 1;
-                T v = (j & 1) ? im[lpos(mm)] : re[lpos(mm)];
-                v *= g;
-                if (KIND == R2R_DST && (i & 1)) v = -v;
-                wr(b, i, v);
+            constexpr int IT = CN > 0 ? ((CN / 2 + CTL - 1) / CTL < 4 ? (CN / 2 + CTL - 1) / CTL : 4) : 2;
+            constexpr T sg = KIND == R2R_DST ? T(-1) : T(1);
+            const int nn = CN > 0 ? CN : N, half = nn / 2, step = CTL > 0 ? CTL : nt;
+            for (int h0 = t; h0 < half; h0 += IT * step) {
+                T x[IT][4];
+#pragma unroll
+                for (int u = 0; u < IT; u++) {
+                    const int h = h0 + u * step, hh = nn - 1 - h;
+                    if (h >= half) continue;
+                    x[u][0] = re[lpos(h)] * g;
+                    x[u][1] = im[lpos(hh)] * (sg * g);
+                    x[u][2] = im[lpos(h)] * g;
+                    x[u][3] = re[lpos(hh)] * (sg * g);
+                }
+#pragma unroll
+                for (int u = 0; u < IT; u++)
+                    if (h0 + u * step < half) wr4(b, 4 * (h0 + u * step), x[u]);
+            }
+            if constexpr (CN == 0) {
+                if ((N & 1) && t == 0) {
+                    wr(b, n - 2, re[lpos((N - 1) / 2)] * g);
+                    wr(b, n - 1, im[lpos((N - 1) / 2)] * (sg * g));
+                }
             }
         }
     }

@@ -65,3 +65,26 @@ def test_columns(orc, n, prec):
         assert e <= tol(n * cols, prec), (n, cols, e)
         p.complexInverse(a, True)
         assert rel(a, x) <= 2 * tol(n * cols, prec), (n, cols)
+
+
+R2R2 = {"dct": (jt.DoubleDCT_2D, jt.FloatDCT_2D), "dst": (jt.DoubleDST_2D, jt.FloatDST_2D),
+        "dht": (jt.DoubleDHT_2D, jt.FloatDHT_2D)}
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("kind", ["dct", "dst", "dht"])
+@pytest.mark.parametrize("dims", [(4, 6), (6, 4), (8, 10), (10, 14), (18, 512), (1024, 6), (30, 32), (64, 22)])
+def test_r2r_quads(orc, kind, dims, prec):
+    """The real transforms read and write four elements at a time: half
+    lengths that are odd leave a pair, with contiguous and strided lines."""
+    x = orc.jrandom_doubles(dims[0], dims[0] * dims[1]).astype(DT[prec])
+    p = R2R2[kind][prec == "f32"](*dims)
+    for fwd in (True, False):
+        scale = kind != "dht" or not fwd
+        a = x.copy()
+        if fwd:
+            p.forward(a, *([True] if kind != "dht" else []))
+        else:
+            p.inverse(a, True)
+        e = rel(a, orc.realnd(kind, list(dims), x.astype(np.float64), fwd, scale))
+        assert e <= tol(x.size, prec), (fwd, e)
