@@ -311,12 +311,16 @@ struct Fft1D {
     int64_t n1 = 0, n2 = 0;
     std::unique_ptr<Fft1D<T>> p1, p2;
     DevBuf hi, lo;
-    // Bluestein
+    // Bluestein: pm is the convolution's plan (a runtime-radix one if m fits
+    // one workgroup's LDS); if it takes the three-pass form (m = n1*n2 with
+    // both single-kernel), pa and pb are runtime-radix plans of n1 and n2
     int64_t m = 0;
-    std::unique_ptr<Fft1D<T>> pm;
+    std::unique_ptr<Fft1D<T>> pm, pa, pb;
     DevBuf chirp, bspec;
 
     bool single() const { return kind == K_TPL || kind == K_GEN; }
+    // Bluestein in one launch, on lines of any stride
+    bool blue_single() const { return kind == K_BLUE && pm->kind == K_GEN; }
     // workspace (complex elements) for `lines` contiguous lines
     int64_t workspace(int64_t lines) const {
         if (kind == K_FOUR) return lines * n + (p2->single() ? 0 : p2->workspace(lines * n1));
@@ -325,6 +329,27 @@ struct Fft1D {
     }
 };
 
+// The runtime-radix plan of a smooth n <= gen_max.
+template <typename T>
+std::unique_ptr<Fft1D<T>> make_gen(int64_t n) {
+    auto p = std::make_unique<Fft1D<T>>();
+    p->n = n;
+    p->kind = K_GEN;
+    p->radices = gen_radices(n);
+    std::vector<int> offs;
+    upload(p->tw, stage_twiddles_gen<T>(p->radices, &offs));
+    GenPlan& g = p->gp;
+    g.n = (int)n;
+    g.nst = (int)p->radices.size();
+    int ns = 1;
+    for (int i = 0; i < g.nst; i++) {
+        const int R = p->radices[i], m = (int)(n / R);
+        g.st[i] = GenStage{R, m, ns, offs[i], 1.0f / (float)m, 1.0f / (float)ns};
+        ns *= R;
+    }
+    return p;
+}
+
 template <typename T>
 std::unique_ptr<Fft1D<T>> make_fft1d(int64_t n) {
     auto p = std::make_unique<Fft1D<T>>();
@@ -332,23 +357,8 @@ std::unique_ptr<Fft1D<T>> make_fft1d(int64_t n) {
     std::vector<int> r;
     bool tpl = tpl_radices(n, r);
     if (tpl || (n <= gen_max<T>() && factor_radices(n, r))) {
-        p->kind = tpl ? K_TPL : K_GEN;
-        if (!tpl) {
-            r = gen_radices(n);
-            std::vector<int> offs;
-            upload(p->tw, stage_twiddles_gen<T>(r, &offs));
-            p->radices = r;
-            GenPlan& g = p->gp;
-            g.n = (int)n;
-            g.nst = (int)r.size();
-            int ns = 1;
-            for (size_t i = 0; i < r.size(); i++) {
-                const int m = (int)(n / r[i]);
-                g.st[i] = GenStage{r[i], m, ns, offs[i], 1.0f / (float)m, 1.0f / (float)ns};
-                ns *= r[i];
-            }
-            return p;
-        }
+        if (!tpl) return make_gen<T>(n);
+        p->kind = K_TPL;
         p->radices = r;
         std::vector<cpx<T>> tab = stage_twiddles<T>(r, nullptr);
         if (n == 4096) {
@@ -403,7 +413,11 @@ std::unique_ptr<Fft1D<T>> make_fft1d(int64_t n) {
     // Bluestein (DoubleFFT_1D.java:1864-2107): chirp c_j = exp(i pi (j^2 mod 2n)/n)
     p->kind = K_BLUE;
     p->m = next_smooth(2 * n - 1);
-    p->pm = make_fft1d<T>(p->m);
+    p->pm = p->m <= gen_max<T>() ? make_gen<T>(p->m) : make_fft1d<T>(p->m);
+    if (p->pm->kind == K_FOUR && p->pm->p2->single()) {
+        p->pa = make_gen<T>(p->pm->n1);
+        p->pb = make_gen<T>(p->pm->n2);
+    }
     std::vector<cpx<T>> ch(n);
     std::vector<long double> br(p->m, 0.0L), bi(p->m, 0.0L);
     const long double PI = 3.141592653589793238462643383279502884L;
@@ -425,7 +439,9 @@ std::unique_ptr<Fft1D<T>> make_fft1d(int64_t n) {
     }
     host_fft_ld(br, bi, -1);
     std::vector<cpx<T>> bs(p->m);
-    for (int64_t i = 0; i < p->m; i++) bs[i] = cpx<T>{(T)(br[i] / p->m), (T)(bi[i] / p->m)};
+    const int64_t n1 = p->pb ? p->pm->n1 : 1, n2 = p->m / n1;
+    for (int64_t i = 0; i < p->m; i++)  // [k1][k2] of k = k1 + n1*k2
+        bs[(i % n1) * n2 + i / n1] = cpx<T>{(T)(br[i] / p->m), (T)(bi[i] / p->m)};
     upload(p->chirp, ch);
     upload(p->bspec, bs);
     return p;
@@ -493,7 +509,7 @@ template <typename T, int DIR, int N, int TL0, bool COL, class IO, int... Rs>
 void go_tpl(IO io, const cpx<T>* tw, hipStream_t st) {
     // LDS hooks, or a store that computes twiddles (four-step pass A), keep
     // the narrower shape: their extra registers would spill
-    constexpr bool HOOKS = IO::pre_lds || IO::post_lds || std::is_same<IO, IOFourA<T, DIR>>::value;
+    constexpr bool HOOKS = IO::pre_lds || IO::post_lds || IO::store_loads;
     constexpr int TL = line_threads<T, N, TL0, COL, HOOKS>();
     constexpr bool REAL = io_real_lines<IO>::value;
     using S = TplShape<T, N, TL, COL, HOOKS, false>;
@@ -808,6 +824,14 @@ void c2c_mapped(const Fft1D<T>& p, const cpx<T>* in, cpx<T>* out, LineMap lm, T 
     }
 }
 
+// One-launch Bluestein transforms of the lines lm.
+template <typename T, int DIR>
+void blue_mapped(const Fft1D<T>& p, const cpx<T>* in, cpx<T>* out, LineMap lm, T scale, hipStream_t st) {
+    const Chirp<T> c{p.chirp.template as<cpx<T>>(), p.bspec.template as<cpx<T>>(), p.n, T(DIR)};
+    IOBlue<T> io{in, out, c, lm, lm.nlines, scale, lm.es != 1};
+    go_gen<T, -1>(*p.pm, io, lm.es != 1, st);
+}
+
 template <typename T, int DIR>
 void c2c_contig(const Fft1D<T>& p, const cpx<T>* in, cpx<T>* out, int64_t lines, T scale,
                 cpx<T>* ws, hipStream_t st) {
@@ -844,6 +868,21 @@ void c2c_contig(const Fft1D<T>& p, const cpx<T>* in, cpx<T>* out, int64_t lines,
         return;
     }
     // Bluestein
+    if (p.blue_single()) {
+        blue_mapped<T, DIR>(p, in, out, LineMap{lines, lines, p.n, 0, 1}, scale, st);
+        return;
+    }
+    if (p.pb) {
+        const Fft1D<T>& f = *p.pm;
+        const Chirp<T> c{p.chirp.template as<cpx<T>>(), p.bspec.template as<cpx<T>>(), p.n, T(DIR)};
+        const cpx<T>* hi = f.hi.template as<cpx<T>>();
+        const cpx<T>* lo = f.lo.template as<cpx<T>>();
+        go_gen<T, -1>(*p.pa, IOBlueL<T, 1>{in, out, ws, c, hi, lo, lines * f.n2, f.n1, f.n2, scale, true}, true, st);
+        go_gen<T, -1>(*p.pb, IOBlueL<T, 2>{in, out, ws, c, hi, lo, lines * f.n1, f.n1, f.n2, scale, false}, false, st);
+        go_gen<T, 1>(*p.pa, IOBlueL<T, 3>{in, out, ws, c, hi, lo, lines * f.n2, f.n1, f.n2, scale, true}, true, st);
+        return;
+    }
+    // a convolution beyond two levels
     cpx<T>* y = ws;
     cpx<T>* ws2 = ws + lines * p.m;
     const cpx<T>* ch = p.chirp.template as<cpx<T>>();
@@ -870,6 +909,7 @@ void c2c_contig(const Fft1D<T>& p, const cpx<T>* in, cpx<T>* out, int64_t lines,
 // kernels compile in parallel.
 #define JT_C2C_INST(X, T, D)                                                                                     \
     X template void c2c_mapped<T, D>(const Fft1D<T>&, const cpx<T>*, cpx<T>*, LineMap, T, hipStream_t, int);       \
+    X template void blue_mapped<T, D>(const Fft1D<T>&, const cpx<T>*, cpx<T>*, LineMap, T, hipStream_t);           \
     X template void c2c_contig<T, D>(const Fft1D<T>&, const cpx<T>*, cpx<T>*, int64_t, T, cpx<T>*, hipStream_t);
 JT_C2C_INST(extern, float, -1)
 JT_C2C_INST(extern, float, 1)

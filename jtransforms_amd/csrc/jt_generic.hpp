@@ -143,7 +143,9 @@ constexpr int gen_butterflies(int R) { return GEN_PTS / R > 0 ? GEN_PTS / R : 1;
 // LDS.  TOG: the outputs go through io.store; else to LDS, in place (all
 // inputs are in registers before the barrier that precedes the first write;
 // the host sizes NT so that gen_butterflies(R) per thread cover the stage).
-template <int R, int DIR, bool FROMG, bool TOG, typename T, class IO>
+// SPEC: each output k is multiplied by io.spec(line, k) and conjugated (the
+// middle of a convolution).
+template <int R, int DIR, bool FROMG, bool TOG, bool SPEC, typename T, class IO>
 __device__ __forceinline__ void gen_stage(const IO& io, GenStage S, int W, int lgW, int pitch, bool col,
                                           const cpx<T>* __restrict__ tw, T* re, T* im, int64_t line0, int nl,
                                           int tid) {
@@ -203,7 +205,7 @@ __device__ __forceinline__ void gen_stage(const IO& io, GenStage S, int W, int l
                     // a store that loads factors of its own: a few at a time,
                     // or their registers spill
                     if constexpr (IO::store_loads)
-                        if (r % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+                        if (sizeof(T) == 8 || r % 2 == 1) __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
                 T* lr = re + ww[b] * pitch;
@@ -212,6 +214,11 @@ __device__ __forceinline__ void gen_stage(const IO& io, GenStage S, int W, int l
 #pragma unroll
                 for (int r = 0; r < R; r++) {
                     const int k = gpos(d + r * ns);
+                    if constexpr (SPEC) {
+                        const cpx<T> p = cmul(v[b][r], io.spec(line0 + ww[b], d, r * ns));
+                        v[b][r] = cpx<T>{p.x, -p.y};
+                        if (sizeof(T) == 8 || r % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+                    }
                     lr[k] = v[b][r].x;
                     li[k] = v[b][r].y;
                 }
@@ -220,7 +227,7 @@ __device__ __forceinline__ void gen_stage(const IO& io, GenStage S, int W, int l
     }
 }
 
-template <int DIR, bool FROMG, bool TOG, typename T, class IO>
+template <int DIR, bool FROMG, bool TOG, bool SPEC = false, typename T, class IO>
 __device__ __forceinline__ void gen_stage_rt(const IO& io, GenStage S, int W, int lgW, int pitch, bool col,
                                              const cpx<T>* __restrict__ tw, T* re, T* im, int64_t line0, int nl,
                                              int tid) {
@@ -229,7 +236,7 @@ __device__ __forceinline__ void gen_stage_rt(const IO& io, GenStage S, int W, in
     asm volatile("" : "+v"(tid));
     switch (S.radix) {
 #define JT_GEN_CASE(R) \
-    case R: gen_stage<R, DIR, FROMG, TOG>(io, S, W, lgW, pitch, col, tw, re, im, line0, nl, tid); break;
+    case R: gen_stage<R, DIR, FROMG, TOG, SPEC>(io, S, W, lgW, pitch, col, tw, re, im, line0, nl, tid); break;
         JT_GEN_CASE(2)
         JT_GEN_CASE(3)
         JT_GEN_CASE(4)
@@ -264,7 +271,10 @@ __device__ __forceinline__ int64_t xcd_group(int64_t bid, int64_t ngroups) {
 // IO contract as for stockham_kernel, except that loads and stores name the
 // element as j + rm with rm uniform over the workgroup; pre/post hooks work on
 // one line with the threads (t, nt) of that line and address LDS through
-// gpos(k).
+// gpos(k).  A policy with conv = true runs the transform twice with the
+// spectrum product between: out = DFT(conj(spec * DFT(in))), i.e. a cyclic
+// convolution up to a conjugation that its store undoes, in one LDS residency
+// (nst >= 2).
 template <typename T, int DIR, class IO>
 __global__ void __launch_bounds__(1024) generic_kernel(IO io, const cpx<T>* __restrict__ tw, GenPlan P) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -300,6 +310,15 @@ __global__ void __launch_bounds__(1024) generic_kernel(IO io, const cpx<T>* __re
         const cpx<T> x = io.load(io.base(line0 + tid), 0, 0);
         re[tid * P.pitch] = x.x;
         im[tid * P.pitch] = x.y;
+    }
+    if constexpr (IO::conv) {
+        for (; s < P.nst - 1; s++) {
+            __syncthreads();
+            gen_stage_rt<DIR, false, false>(io, P.st[s], W, P.lgW, P.pitch, P.col, tw, re, im, line0, nl, tid);
+        }
+        __syncthreads();
+        gen_stage_rt<DIR, false, false, true>(io, P.st[s], W, P.lgW, P.pitch, P.col, tw, re, im, line0, nl, tid);
+        s = 0;
     }
     const int inner = IO::post_lds ? P.nst : P.nst - 1;
     for (; s < inner; s++) {

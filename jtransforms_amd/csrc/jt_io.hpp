@@ -48,7 +48,7 @@ enum { NT_LOAD = 1, NT_STORE = 2 };
 // kernels registers and load batching.
 template <typename T, int NT = 0>
 struct IOStrided {
-    static constexpr bool pre_lds = false, post_lds = false, store_loads = false;
+    static constexpr bool pre_lds = false, post_lds = false, store_loads = false, conv = false;
     static constexpr int streaming = NT;
     static const char* tag() { return NT == 0 ? "c2c" : "c2c,nt"; }
     std::string desc() const { return ",es=" + std::to_string(m.es); }
@@ -127,7 +127,7 @@ __device__ __forceinline__ cpx<T> tw2(const cpx<T>* __restrict__ hi, const cpx<T
 // follow as columns of that n2 x n1 matrix, or in place (oj = 1, ok = n2).
 template <typename T, int DIR>
 struct IOFourA {
-    static constexpr bool pre_lds = false, post_lds = false, store_loads = true;
+    static constexpr bool pre_lds = false, post_lds = false, store_loads = true, conv = false;
     static const char* tag() { return "fourA"; }
     std::string desc() const { return ",n1=" + std::to_string(n1) + ",n2=" + std::to_string(n2); }
     const cpx<T>* in;
@@ -155,6 +155,114 @@ struct IOFourA {
     __device__ void post(int64_t, At, const T*, const T*, int, int) const {}
 };
 
+// Bluestein (DoubleFFT_1D.java:1864-2107): X_k = c'_k * sum_j (x_j c'_j)
+// c_{k-j} with the chirp c_j = exp(i pi j^2/n) and c' its conjugate (forward)
+// or itself (backward, with the conjugated kernel spectrum), as a cyclic
+// convolution of length m >= 2n-1.
+template <typename T>
+struct Chirp {
+    const cpx<T>* ch;  // n entries
+    const cpx<T>* bs;  // kernel spectrum / m, m entries
+    int64_t n;
+    T sg;              // -1 forward, +1 backward
+    __device__ __forceinline__ cpx<T> at(int64_t k) const { return cpx<T>{ch[k].x, sg * ch[k].y}; }
+    // x[k] c'_k, 0 for k >= n; `at_k(k)` loads x[k] (without a branch, so that
+    // all loads of a thread are in flight together)
+    template <class F>
+    __device__ __forceinline__ cpx<T> premul(int64_t k, F at_k) const {
+        const bool in = k < n;
+        const int64_t kk = in ? k : n - 1;
+        const cpx<T> v = cmul(at_k(kk), at(kk));
+        return in ? v : cpx<T>{T(0), T(0)};
+    }
+    __device__ __forceinline__ cpx<T> spec(int64_t k) const { return cpx<T>{bs[k].x, -sg * bs[k].y}; }
+    __device__ __forceinline__ cpx<T> postmul(int64_t k, cpx<T> v, T scale) const {
+        const cpx<T> o = cmul(v, at(k));
+        return cpx<T>{o.x * scale, o.y * scale};
+    }
+};
+
+// A whole Bluestein transform per line: the m-point convolution in one LDS
+// residency, so a line is read and written once.  (As five to seven launches
+// with the m points in memory between them, 2123 lines of 606 FP64 points took
+// 133 us a direction, 42 this way; an axis of stride > 1 needs no gather.)
+template <typename T>
+struct IOBlue {
+    static constexpr bool pre_lds = false, post_lds = false, store_loads = true, conv = true;
+    static const char* tag() { return "blue"; }
+    std::string desc() const { return ",n=" + std::to_string(c.n) + ",es=" + std::to_string(m.es); }
+    const cpx<T>* in;
+    cpx<T>* out;
+    Chirp<T> c;
+    LineMap m;
+    int64_t nlines;
+    T scale;
+    bool xcd;
+    __device__ __forceinline__ int64_t base(int64_t l) const { return m.base(l); }
+    __device__ __forceinline__ cpx<T> load(int64_t b, int k, int rm) const {
+        return c.premul(k + rm, [&](int64_t kk) { return in[b + kk * m.es]; });
+    }
+    __device__ __forceinline__ cpx<T> spec(int64_t, int k, int rm) const { return c.spec(k + rm); }
+    __device__ __forceinline__ void store(int64_t b, int k, int rm, cpx<T> v) const {
+        const int64_t kk = k + rm;
+        if (kk < c.n) out[b + kk * m.es] = c.postmul(kk, cpx<T>{v.x, -v.y}, scale);
+    }
+};
+
+// Longer convolutions, m = n1*n2, in three passes over an n1 x n2 matrix in
+// the workspace: the premultiplied, zero-padded columns (FFT over n1, times
+// exp(-2 pi i j2 k1/m)); the rows (FFT over n2, spectrum product, inverse FFT,
+// times exp(+2 pi i j2 k1/m), in place); the columns back, postmultiplied.
+// Three launches instead of seven: one transform of 10158 FP64 points, which
+// waits for launches and not for memory, 40.5 -> 26 us.
+// The spectrum is stored in the order the rows meet it, [k1][k2].
+template <typename T, int PASS>
+struct IOBlueL {
+    static constexpr bool pre_lds = false, post_lds = false, store_loads = true, conv = PASS == 2;
+    static const char* tag() { return PASS == 1 ? "blueA" : PASS == 2 ? "blueB" : "blueC"; }
+    std::string desc() const { return ",n1=" + std::to_string(n1) + ",n2=" + std::to_string(n2); }
+    const cpx<T>* in;
+    cpx<T>* out;
+    cpx<T>* ws;
+    Chirp<T> c;
+    const cpx<T>* hi;
+    const cpx<T>* lo;
+    int64_t nlines, n1, n2;
+    T scale;
+    bool xcd;
+    struct At {
+        int64_t x, w;  // offsets of the transform's data and matrix
+        int64_t q;     // column j2 (passes 1, 3) or row k1 (pass 2)
+    };
+    __device__ __forceinline__ At base(int64_t l) const {
+        const int64_t per = PASS == 2 ? n1 : n2;
+        if (nlines == per) return At{0, 0, l};  // one transform
+        const int64_t b = l / per;
+        return At{b * c.n, b * n1 * n2, l - b * per};
+    }
+    __device__ __forceinline__ cpx<T> load(At a, int k, int rm) const {
+        if constexpr (PASS == 1)
+            return c.premul((a.q + k * n2) + rm * n2, [&](int64_t kk) { return in[a.x + kk]; });
+        else if constexpr (PASS == 2) return ws[(a.w + a.q * n2 + k) + rm];
+        else return ws[(a.w + a.q + k * n2) + rm * n2];
+    }
+    __device__ __forceinline__ cpx<T> spec(int64_t l, int k, int rm) const { return c.spec(l % n1 * n2 + k + rm); }
+    __device__ __forceinline__ void store(At a, int k, int rm, cpx<T> v) const {
+        if constexpr (PASS == 1) {
+            ws[(a.w + a.q + k * n2) + rm * n2] = cmul(v, tw2<-1>(hi, lo, a.q * k + a.q * rm));
+        } else if constexpr (PASS == 2) {
+            ws[(a.w + a.q * n2 + k) + rm] = cmul(cpx<T>{v.x, -v.y}, tw2<1>(hi, lo, a.q * k + a.q * rm));
+        } else {
+            const int64_t kk = (a.q + k * n2) + rm * n2;
+            if (kk < c.n) out[a.x + kk] = c.postmul(kk, v, scale);
+        }
+    }
+    template <int CN, int CTL>
+    __device__ void pre(int64_t, At, T*, T*, int, int) const {}
+    template <int CN, int CTL>
+    __device__ void post(int64_t, At, const T*, const T*, int, int) const {}
+};
+
 // realForward post pass (reference: CommonUtils.rftfsub :5750-5776 and the
 // fold at DoubleFFT_1D.java:543-545).  The line holds the N-point complex FFT
 // Z of the 2N reals taken pairwise; the packed result is
@@ -163,7 +271,7 @@ struct IOFourA {
 // w = exp(-2 pi i/2N).  rtw[k] = w^k for k in [0, N/2].
 template <typename T>
 struct IOR2C {
-    static constexpr bool pre_lds = false, post_lds = true, store_loads = false;
+    static constexpr bool pre_lds = false, post_lds = true, store_loads = false, conv = false;
     static const char* tag() { return "r2c"; }
     std::string desc() const { return ",es=" + std::to_string(m.es); }
     const cpx<T>* in;  // reals viewed as complex pairs
@@ -219,7 +327,7 @@ struct IOR2C {
 // is sum-normalised (x_{2m} + i x_{2m+1}) * 2N, stored times `scale`.
 template <typename T>
 struct IOC2R {
-    static constexpr bool pre_lds = true, post_lds = false, store_loads = false;
+    static constexpr bool pre_lds = true, post_lds = false, store_loads = false, conv = false;
     static const char* tag() { return "c2r"; }
     std::string desc() const { return ",es=" + std::to_string(m.es); }
     const T* in;     // packed reals

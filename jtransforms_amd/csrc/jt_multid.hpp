@@ -38,6 +38,10 @@ void axis_c2c(const Fft1D<T>& p, cpx<T>* data, LineMap lm, T scale, cpx<T>* ws, 
         c2c_mapped<T, DIR>(p, data, data, lm, scale, st);
         return;
     }
+    if (p.blue_single()) {
+        blue_mapped<T, DIR>(p, data, data, lm, scale, st);
+        return;
+    }
     bool contig = lm.es == 1 && lm.s0 == p.n && lm.n0 >= lm.nlines;
     if (contig) {
         c2c_contig<T, DIR>(p, data, data, lm.nlines, scale, ws, st);

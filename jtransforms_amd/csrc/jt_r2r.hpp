@@ -57,7 +57,7 @@ inline R2RScale dct3_scale(int64_t n, bool scale) {
 // ---------------------------------------------------------------------------
 template <typename T, int KIND, bool FWD>
 struct IOR2R {
-    static constexpr bool pre_lds = true, post_lds = true, store_loads = false;
+    static constexpr bool pre_lds = true, post_lds = true, store_loads = false, conv = false;
     // lines of reals: a column group's row segment is W * sizeof(T) bytes
     static constexpr bool real_lines = true;
     static const char* tag() {

@@ -88,3 +88,32 @@ def test_r2r_quads(orc, kind, dims, prec):
             p.inverse(a, True)
         e = rel(a, orc.realnd(kind, list(dims), x.astype(np.float64), fwd, scale))
         assert e <= tol(x.size, prec), (fwd, e)
+
+
+# convolution lengths just inside and outside one workgroup's LDS (4096 points
+# in FP64, 8192 in FP32), short ones, and a two-level one
+BLUE = [(n, p) for p in ("f64", "f32") for n in (17, 19, 34, 67, 519, 1021, 2047, 2051, 4079, 4103)] + [(20011, "f64")]
+
+
+@pytest.mark.parametrize("n,prec", BLUE)
+def test_bluestein(orc, n, prec):
+    """Bluestein lengths as rows of a batch and as columns, both directions."""
+    cls = FFT2[prec]
+    for lines in (1, 3, 70):
+        if n * lines > 1 << 18:
+            continue
+        x = orc.jrandom_doubles(n + lines, 2 * n * lines).astype(DT[prec])
+        rows = jt.FFTBatch1D(n, lines, precision=prec)
+        a = x.copy()
+        rows.complexForward(a)
+        seg = slice(2 * n * (lines - 1), 2 * n * lines)
+        assert rel(a[seg], orc.complex_forward(n, x[seg].astype(np.float64))) <= tol(n, prec), (n, lines)
+        rows.complexInverse(a, True)
+        assert rel(a, x) <= 2 * tol(n, prec), (n, lines)
+    x = orc.jrandom_doubles(n, 2 * n * 6).astype(DT[prec])
+    a = x.copy()
+    p = cls(n, 6)
+    p.complexForward(a)
+    assert rel(a, orc.fftnd_complex([n, 6], x.astype(np.float64), -1)) <= tol(6 * n, prec)
+    p.complexInverse(a, True)
+    assert rel(a, x) <= 2 * tol(6 * n, prec)
