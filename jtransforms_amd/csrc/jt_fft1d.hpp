@@ -329,6 +329,49 @@ struct Fft1D {
     }
 };
 
+// The four-step column length n1 of a smooth n > gen_max, 0 if there is none.
+template <typename T>
+int64_t four_split(int64_t n) {
+    // n1 (column FFT) * n2 (row FFT), both single-kernel
+    int64_t best1 = 0;
+    for (int64_t a = 2; a <= gen_max<T>(); a++) {
+        if (n % a) continue;
+        int64_t b = n / a;
+        if (b > gen_max<T>()) continue;
+        std::vector<int> ra, rb;
+        if (!factor_radices(a, ra) || !factor_radices(b, rb)) continue;
+        // prefer balanced split, n1 a power of two when possible
+        if (!best1 || std::llabs(a - b) < std::llabs(best1 - n / best1)) best1 = a;
+    }
+    if (!best1) {
+        // n beyond gen_max^2: the largest single-kernel n1 whose cofactor
+        // is smooth; the n2-point row FFTs are then a plan of their own
+        // (four-step again), run in place on the workspace
+        for (int64_t a = gen_max<T>(); a >= 2 && !best1; a--) {
+            if (n % a) continue;
+            std::vector<int> ra, rb;
+            if (factor_radices(a, ra) && factor_radices(n / a, rb)) best1 = a;
+        }
+    }
+    return best1;
+}
+
+// Fft1D::workspace of the n-point plan, without building it.
+template <typename T>
+int64_t plan_workspace(int64_t n, int64_t lines) {
+    std::vector<int> r;
+    const bool smooth = factor_radices(n, r);
+    if (n <= gen_max<T>() && smooth) return 0;
+    if (smooth) {
+        if (const int64_t n1 = four_split<T>(n)) {
+            const int64_t n2 = n / n1;
+            return lines * n + (n2 <= gen_max<T>() ? 0 : plan_workspace<T>(n2, lines * n1));
+        }
+    }
+    const int64_t m = next_smooth(2 * n - 1);
+    return lines * m + plan_workspace<T>(m, lines);
+}
+
 // The runtime-radix plan of a smooth n <= gen_max.
 template <typename T>
 std::unique_ptr<Fft1D<T>> make_gen(int64_t n) {
@@ -375,27 +418,7 @@ std::unique_ptr<Fft1D<T>> make_fft1d(int64_t n) {
         return p;
     }
     if (factor_radices(n, r)) {
-        // four-step: n1 (column FFT) * n2 (row FFT), both single-kernel
-        int64_t best1 = 0;
-        for (int64_t a = 2; a <= gen_max<T>(); a++) {
-            if (n % a) continue;
-            int64_t b = n / a;
-            if (b > gen_max<T>()) continue;
-            std::vector<int> ra, rb;
-            if (!factor_radices(a, ra) || !factor_radices(b, rb)) continue;
-            // prefer balanced split, n1 a power of two when possible
-            if (!best1 || std::llabs(a - b) < std::llabs(best1 - n / best1)) best1 = a;
-        }
-        if (!best1) {
-            // n beyond gen_max^2: the largest single-kernel n1 whose cofactor
-            // is smooth; the n2-point row FFTs are then a plan of their own
-            // (four-step again), run in place on the workspace
-            for (int64_t a = gen_max<T>(); a >= 2 && !best1; a--) {
-                if (n % a) continue;
-                std::vector<int> ra, rb;
-                if (factor_radices(a, ra) && factor_radices(n / a, rb)) best1 = a;
-            }
-        }
+        const int64_t best1 = four_split<T>(n);
         if (best1) {
             p->kind = K_FOUR;
             p->n1 = best1;

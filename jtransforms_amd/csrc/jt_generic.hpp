@@ -311,26 +311,27 @@ __global__ void __launch_bounds__(1024) generic_kernel(IO io, const cpx<T>* __re
         re[tid * P.pitch] = x.x;
         im[tid * P.pitch] = x.y;
     }
-    if constexpr (IO::conv) {
-        for (; s < P.nst - 1; s++) {
-            __syncthreads();
-            gen_stage_rt<DIR, false, false>(io, P.st[s], W, P.lgW, P.pitch, P.col, tw, re, im, line0, nl, tid);
-        }
-        __syncthreads();
-        gen_stage_rt<DIR, false, false, true>(io, P.st[s], W, P.lgW, P.pitch, P.col, tw, re, im, line0, nl, tid);
-        s = 0;
-    }
-    const int inner = IO::post_lds ? P.nst : P.nst - 1;
+    // (one loop over both transforms of a convolution: with two, the compiler
+    // keeps a copy of the stage list in scratch)
+    const int all = IO::conv ? 2 * P.nst : P.nst;
+    const int inner = IO::post_lds ? all : all - 1;
     for (; s < inner; s++) {
+        const GenStage S = P.st[IO::conv && s >= P.nst ? s - P.nst : s];
         __syncthreads();
-        gen_stage_rt<DIR, false, false>(io, P.st[s], W, P.lgW, P.pitch, P.col, tw, re, im, line0, nl, tid);
+        if constexpr (IO::conv) {
+            if (s == P.nst - 1) {
+                gen_stage_rt<DIR, false, false, true>(io, S, W, P.lgW, P.pitch, P.col, tw, re, im, line0, nl, tid);
+                continue;
+            }
+        }
+        gen_stage_rt<DIR, false, false>(io, S, W, P.lgW, P.pitch, P.col, tw, re, im, line0, nl, tid);
     }
     __syncthreads();
     if constexpr (IO::post_lds) {
         if (hw < nl)
             io.template post<0, 0>(line0 + hw, io.base(line0 + hw), re + hw * P.pitch, im + hw * P.pitch, ht, hn);
-    } else if (s < P.nst) {
-        gen_stage_rt<DIR, false, true>(io, P.st[s], W, P.lgW, P.pitch, P.col, tw, re, im, line0, nl, tid);
+    } else if (s < all) {
+        gen_stage_rt<DIR, false, true>(io, P.st[P.nst - 1], W, P.lgW, P.pitch, P.col, tw, re, im, line0, nl, tid);
     } else {
         // one stage at most: the results are in LDS
         for (int idx = tid; idx < nl * P.n; idx += blockDim.x) {

@@ -1,0 +1,6 @@
+// FP64 real transforms that run two lines as one complex transform.
+#include "jt_pair.hpp"
+
+namespace jt {
+JT_PAIR_INST(, double)
+}  // namespace jt

@@ -14,14 +14,13 @@
 // (v_j = x_2j, v_{n-1-j} = x_{2j+1}) into n/2 complex points, the post hook
 // applies the real-FFT split and the exp(-i pi k/2n) twiddle and stores the
 // n results (with the DST's sign/reverse maps folded into the index maps).
-// Other lengths use a mirrored 2n-point complex transform (the reference's
-// own non-power-of-two DCT route, DoubleDCT_1D.java:195-242).
+// Odd n, and even n whose Bluestein convolution fits LDS, run two lines as one
+// n-point complex transform (jt_pair.hpp); other even n the same steps as the
+// fused form, around an n/2-point transform of several launches.
 #pragma once
 #include "jt_multid.hpp"
 
 namespace jt {
-
-enum { R2R_DCT = 1, R2R_DST = 2, R2R_DHT = 3 };
 
 // ---------------------------------------------------------------------------
 // scale conventions
@@ -43,6 +42,45 @@ inline R2RScale dct3_scale(int64_t n, bool scale) {
     if (scale) return {std::sqrt(2.0), std::sqrt(2.0 / (double)n)};
     if (is_pow2(n)) return {2.0, 1.0};
     return {1.0, 1.0 / (double)n};
+}
+
+// ---------------------------------------------------------------------------
+// the split between the n/2-point complex transform Z and the outputs at k,
+// n-k, N-k and N+k (N = n/2, 0 < k <= N/2); w = exp(-2 pi i k/n), qa = q_k,
+// qb = q_{N-k}, q_k = exp(-i pi k/2n)
+// ---------------------------------------------------------------------------
+template <int KIND, typename T>
+__device__ __forceinline__ void half_fwd(cpx<T> A, cpx<T> B, cpx<T> w, cpx<T> qa, cpx<T> qb, T* y) {
+    // A = Z_k, B = conj Z_{N-k}
+    const cpx<T> fe = cadd(A, B), d = csub(A, B);
+    const cpx<T> fo = {d.y, -d.x};
+    const cpx<T> wf = cmul(w, fo);
+    const cpx<T> Vk = {(fe.x + wf.x) * T(0.5), (fe.y + wf.y) * T(0.5)};
+    const cpx<T> Vc = {(fe.x - wf.x) * T(0.5), -(fe.y - wf.y) * T(0.5)};  // V_{N-k}
+    if constexpr (KIND == R2R_DHT) {
+        y[0] = Vk.x - Vk.y;
+        y[1] = Vk.x + Vk.y;
+        y[2] = Vc.x - Vc.y;
+        y[3] = Vc.x + Vc.y;
+    } else {
+        const cpx<T> a = cmul(qa, Vk), c = cmul(qb, Vc);
+        y[0] = a.x;
+        y[1] = -a.y;
+        y[2] = c.x;
+        y[3] = -c.y;
+    }
+}
+// DCT-III: Z_k and Z_{N-k} from V_k = conj(q_k)(a_k - i a_{n-k}) and V_{N-k}
+template <typename T>
+__device__ __forceinline__ void half_inv(cpx<T> qa, cpx<T> qb, cpx<T> w, T ak, T ank, T akk, T ankk, cpx<T>& Zk,
+                                         cpx<T>& Zkk) {
+    const cpx<T> Vk = cmulc(cpx<T>{ak, -ank}, qa);
+    const cpx<T> Vc = cmulc(cpx<T>{akk, -ankk}, qb);
+    const cpx<T> Xc = {Vc.x, -Vc.y};  // conj V_{N-k}
+    const cpx<T> E = cadd(Vk, Xc), D = csub(Vk, Xc);
+    const cpx<T> O = cmul(D, cpx<T>{w.x, -w.y});
+    Zk = cpx<T>{E.x - O.y, E.y + O.x};
+    Zkk = cpx<T>{E.x + O.y, O.x - E.y};
 }
 
 // ---------------------------------------------------------------------------
@@ -132,18 +170,14 @@ struct IOR2R {
     }
     // inverse: Z_k, Z_{N-k} from a'_k, a'_{n-k}, a'_{N-k}, a'_{N+k}
     __device__ __forceinline__ void inv_pair(int k, T ak, T ank, T akk, T ankk, T* re, T* im) const {
-        int kk = N - k;
-        cpx<T> Vk = cmulc(cpx<T>{ak, -ank}, q[k]);
-        cpx<T> Vc = cmulc(cpx<T>{akk, -ankk}, q[kk]);
-        cpx<T> Xc = {Vc.x, -Vc.y};  // conj V_{N-k}
-        cpx<T> E = cadd(Vk, Xc), D = csub(Vk, Xc);
-        cpx<T> w = {rtw[k].x, -rtw[k].y};
-        cpx<T> O = cmul(D, w);
-        re[lpos(k)] = E.x - O.y;
-        im[lpos(k)] = E.y + O.x;
+        const int kk = N - k;
+        cpx<T> Zk, Zkk;
+        half_inv(q[k], q[kk], rtw[k], ak, ank, akk, ankk, Zk, Zkk);
+        re[lpos(k)] = Zk.x;
+        im[lpos(k)] = Zk.y;
         if (kk != k) {
-            re[lpos(kk)] = E.x + O.y;
-            im[lpos(kk)] = O.x - E.y;
+            re[lpos(kk)] = Zkk.x;
+            im[lpos(kk)] = Zkk.y;
         }
     }
 
@@ -241,23 +275,7 @@ struct IOR2R {
                     const int kk = nn - k;
                     cpx<T> A = {re[lpos(k)], im[lpos(k)]};
                     cpx<T> B = {re[lpos(kk)], -im[lpos(kk)]};
-                    cpx<T> fe = cadd(A, B), d = csub(A, B);
-                    cpx<T> fo = {d.y, -d.x};
-                    cpx<T> wf = cmul(w[u], fo);
-                    cpx<T> Vk = {(fe.x + wf.x) * T(0.5), (fe.y + wf.y) * T(0.5)};
-                    cpx<T> Vc = {(fe.x - wf.x) * T(0.5), -(fe.y - wf.y) * T(0.5)};  // V_{N-k}
-                    if constexpr (KIND == R2R_DHT) {
-                        y[u][0] = Vk.x - Vk.y;
-                        y[u][1] = Vk.x + Vk.y;
-                        y[u][2] = Vc.x - Vc.y;
-                        y[u][3] = Vc.x + Vc.y;
-                    } else {
-                        cpx<T> a = cmul(qa[u], Vk), c = cmul(qb[u], Vc);
-                        y[u][0] = a.x;
-                        y[u][1] = -a.y;
-                        y[u][2] = c.x;
-                        y[u][3] = -c.y;
-                    }
+                    half_fwd<KIND>(A, B, w[u], qa[u], qb[u], y[u]);
                 }
 #pragma unroll
                 for (int u = 0; u < IT; u++) {
@@ -302,62 +320,77 @@ struct IOR2R {
 };
 
 // ---------------------------------------------------------------------------
-// fallback kernels (any n): through a complex transform of length 2n (DCT,
-// DST) or n (DHT) on gathered lines
+// the same steps for even n whose n/2-point transform takes several launches:
+// lines gathered to N complex points each in the workspace, and back
 // ---------------------------------------------------------------------------
+template <int KIND>
+__device__ __forceinline__ int64_t half_vidx(int64_t j, int64_t n) {
+    if (KIND == R2R_DHT) return j;
+    return 2 * j < n ? 2 * j : 2 * (n - 1 - j) + 1;
+}
+
 template <typename T, int KIND, bool FWD>
-__global__ void r2r_fb_pre(const T* __restrict__ x, cpx<T>* __restrict__ y, LineMap m, int64_t n,
-                           int64_t L, const cpx<T>* __restrict__ q, T f0) {
-    // L = complex length per line (2n or n)
+__global__ void half_in(const T* __restrict__ x, cpx<T>* __restrict__ z, LineMap m, int64_t n,
+                        const cpx<T>* __restrict__ q, const cpx<T>* __restrict__ rtw, T f0) {
+    const int64_t N = n / 2, per = FWD ? N : N / 2 + 1;
     int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    for (; i < m.nlines * L; i += (int64_t)gridDim.x * blockDim.x) {
-        int64_t l = i / L, j = i % L;
-        int64_t b = m.base(l);
-        cpx<T> v{T(0), T(0)};
-        if (KIND == R2R_DHT) {
-            v.x = x[b + j * m.es];
-        } else if (FWD) {
-            int64_t src = j < n ? j : 2 * n - 1 - j;  // mirrored extension
-            T xv = x[b + src * m.es];
-            if (KIND == R2R_DST && (src & 1)) xv = -xv;
-            v.x = xv;
+    for (; i < m.nlines * per; i += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t l = i / per, k = i - l * per, b = m.base(l);
+        cpx<T>* zl = z + l * N;
+        auto rd = [&](int64_t j) { return x[b + j * m.es]; };
+        if constexpr (FWD) {
+            const int64_t j0 = half_vidx<KIND>(2 * k, n), j1 = half_vidx<KIND>(2 * k + 1, n);
+            const T v0 = rd(j0), v1 = rd(j1);
+            zl[k] = cpx<T>{KIND == R2R_DST && (j0 & 1) ? -v0 : v0, KIND == R2R_DST && (j1 & 1) ? -v1 : v1};
         } else {
-            // u_k = c_k a'_k exp(+i pi k/2n), k < n; zero above
-            if (j < n) {
-                int64_t kk = KIND == R2R_DST ? n - 1 - j : j;
-                T a = x[b + kk * m.es];
-                T c = j == 0 ? T(0.5) * f0 : T(1);
-                cpx<T> w = {q[j].x, -q[j].y};
-                v = cpx<T>{a * c * w.x, a * c * w.y};
+            auto a = [&](int64_t j) { return rd(KIND == R2R_DST ? n - 1 - j : j); };
+            if (k == 0) {
+                const T v0 = a(0) * f0, vN = T(1.41421356237309504880168872420970) * a(N);
+                zl[0] = cpx<T>{v0 + vN, v0 - vN};
+                continue;
             }
+            cpx<T> Zk, Zkk;
+            half_inv(q[k], q[N - k], rtw[k], a(k), a(n - k), a(N - k), a(N + k), Zk, Zkk);
+            zl[k] = Zk;
+            if (N - k != k) zl[N - k] = Zkk;
         }
-        y[i] = v;
     }
 }
 
 template <typename T, int KIND, bool FWD>
-__global__ void r2r_fb_post(const cpx<T>* __restrict__ y, T* __restrict__ x, LineMap m, int64_t n,
-                            int64_t L, const cpx<T>* __restrict__ q, T f0, T g) {
+__global__ void half_out(const cpx<T>* __restrict__ z, T* __restrict__ x, LineMap m, int64_t n,
+                         const cpx<T>* __restrict__ q, const cpx<T>* __restrict__ rtw, T f0, T g) {
+    const int64_t N = n / 2, per = FWD ? N / 2 + 1 : N;
     int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    for (; i < m.nlines * n; i += (int64_t)gridDim.x * blockDim.x) {
-        int64_t l = i / n, k = i % n;
-        int64_t b = m.base(l);
-        const cpx<T>* yl = y + l * L;
-        T v;
-        if (KIND == R2R_DHT) {
-            v = (yl[k].x - yl[k].y) * g;
-            x[b + k * m.es] = v;
-        } else if (FWD) {
-            // DFT_2n(mirror) = 2 exp(i pi k/2n) C_k
-            cpx<T> u = cmul(q[k], yl[k]);
-            v = T(0.5) * u.x * g;
-            if (k == 0) v *= f0;
-            int64_t dst = KIND == R2R_DST ? n - 1 - k : k;
-            x[b + dst * m.es] = v;
+    for (; i < m.nlines * per; i += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t l = i / per, k = i - l * per, b = m.base(l);
+        const cpx<T>* zl = z + l * N;
+        if constexpr (FWD) {
+            auto wr = [&](int64_t j, T v) { x[b + (KIND == R2R_DST ? n - 1 - j : j) * m.es] = v * g; };
+            if (k == 0) {
+                const T s = zl[0].x + zl[0].y, d = zl[0].x - zl[0].y;
+                wr(0, KIND == R2R_DHT ? s : s * f0);
+                wr(N, KIND == R2R_DHT ? d : T(0.70710678118654752440084436210485) * d);
+                continue;
+            }
+            T y[4];
+            cpx<T> qa{}, qb{};
+            if constexpr (KIND != R2R_DHT) {
+                qa = q[k];
+                qb = q[N - k];
+            }
+            half_fwd<KIND>(zl[k], cpx<T>{zl[N - k].x, -zl[N - k].y}, rtw[k], qa, qb, y);
+            wr(k, y[0]);
+            wr(n - k, y[1]);
+            if (N - k != k) {
+                wr(N - k, y[2]);
+                wr(N + k, y[3]);
+            }
         } else {
-            v = yl[k].x * g * T(2);
-            if (KIND == R2R_DST && (k & 1)) v = -v;
-            x[b + k * m.es] = v;
+            const int64_t j0 = half_vidx<KIND>(2 * k, n), j1 = half_vidx<KIND>(2 * k + 1, n);
+            const T v0 = zl[k].x * g, v1 = zl[k].y * g;
+            x[b + j0 * m.es] = KIND == R2R_DST && (j0 & 1) ? -v0 : v0;
+            x[b + j1 * m.es] = KIND == R2R_DST && (j1 & 1) ? -v1 : v1;
         }
     }
 }
@@ -424,14 +457,17 @@ template <typename T>
 struct R2R1D {
     int kind = R2R_DCT;
     int64_t n = 0;
-    std::unique_ptr<Fft1D<T>> half;  // n/2, fused path
-    std::unique_ptr<Fft1D<T>> big;   // 2n (DCT/DST) or n (DHT), fallback
+    std::unique_ptr<Fft1D<T>> half;  // n/2: fused if one launch, else through the workspace
+    std::unique_ptr<Fft1D<T>> full;  // n: lines in pairs
     DevBuf q, rtw;
     bool fused() const { return half && half->single(); }
-    int64_t L() const { return kind == R2R_DHT ? n : 2 * n; }
     int64_t ws_elems(int64_t lines) const {
         if (fused() || n == 1) return 0;
-        return lines * L() + big->workspace(lines);
+        // the bound that callers of the fixed-scratch entry point know: the
+        // workspace of a 2n-point (DHT: n-point) complex transform of each line
+        const int64_t L = kind == R2R_DHT ? n : 2 * n, pairs = (lines + 1) / 2;
+        const int64_t need = half ? lines * (n / 2) + half->workspace(lines) : pairs * n + full->workspace(pairs);
+        return std::max(need, lines * L + plan_workspace<T>(L, lines));
     }
 };
 
@@ -446,7 +482,7 @@ std::unique_ptr<R2R1D<T>> make_r2r1d(int family, int64_t n) {
     upload(r->q, q);
     if (n % 2 == 0 && n >= 4) {
         auto h = make_fft1d<T>(n / 2);
-        if (h->single()) {
+        if (h->single() || next_smooth(2 * n - 1) > gen_max<T>()) {
             r->half = std::move(h);
             std::vector<cpx<T>> w(n / 4 + 2);
             for (int64_t k = 0; k < (int64_t)w.size(); k++) w[k] = expm<T>(k, n);
@@ -454,7 +490,7 @@ std::unique_ptr<R2R1D<T>> make_r2r1d(int family, int64_t n) {
             return r;
         }
     }
-    r->big = make_fft1d<T>(r->L());
+    r->full = make_fft1d<T>(n);
     return r;
 }
 
@@ -474,22 +510,24 @@ void r2r_axis_k(const R2R1D<T>& r, T* data, LineMap lm, bool scale, cpx<T>* ws, 
         else run_single<T, (FWD || KIND == R2R_DHT) ? -1 : 1, true>(*r.half, io, st);
         return;
     }
-    const int64_t L = r.L();
-    cpx<T>* y = ws;
-    cpx<T>* ws2 = ws + lm.nlines * L;
-    { JT_PROF(st, "r2r_fb_pre");
-    hipLaunchKernelGGL((r2r_fb_pre<T, KIND, FWD>), ew_grid(lm.nlines * L), dim3(256), 0, st, data, y, lm, n, L,
-                       r.q.template as<cpx<T>>(), T(sc.f0));
+    // inverse: as above for the n-point and the half-length form alike
+    const T f0 = T(sc.f0), g = FWD || KIND == R2R_DHT ? T(sc.g) : T(sc.g * 0.5);
+    const cpx<T>* q = r.q.template as<cpx<T>>();
+    if (r.full) {
+        pair_lines<T, KIND, FWD>(*r.full, data, q, lm, f0, g, ws, st);
+        return;
+    }
+    const cpx<T>* rtw = r.rtw.template as<cpx<T>>();
+    const int64_t N = n / 2;
+    constexpr int D = FWD || KIND == R2R_DHT ? -1 : 1;
+    { JT_PROF(st, "half_in");
+    hipLaunchKernelGGL((half_in<T, KIND, FWD>), ew_grid(lm.nlines * N), dim3(256), 0, st, data, ws, lm, n, q, rtw, f0);
     }
     JT_HIP(hipGetLastError());
-    if (KIND == R2R_DHT || FWD) c2c_contig<T, -1>(*r.big, y, y, lm.nlines, T(1), ws2, st);
-    else c2c_contig<T, 1>(*r.big, y, y, lm.nlines, T(1), ws2, st);
-    // inverse: backward 2n sum of u gives y(a') directly (the 1/2 on a_0 is
-    // in u_0): fb_post multiplies by 2*g*0.5 -> use g/2 here
-    T gpost = (KIND == R2R_DHT || FWD) ? T(sc.g) : T(sc.g * 0.5);
-    { JT_PROF(st, "r2r_fb_post");
-    hipLaunchKernelGGL((r2r_fb_post<T, KIND, FWD>), ew_grid(lm.nlines * n), dim3(256), 0, st, y, data, lm, n, L,
-                       r.q.template as<cpx<T>>(), T(sc.f0), gpost);
+    c2c_contig<T, D>(*r.half, ws, ws, lm.nlines, T(1), ws + lm.nlines * N, st);
+    { JT_PROF(st, "half_out");
+    hipLaunchKernelGGL((half_out<T, KIND, FWD>), ew_grid(lm.nlines * N), dim3(256), 0, st, ws, data, lm, n, q, rtw, f0,
+                       g);
     }
     JT_HIP(hipGetLastError());
 }

@@ -3,6 +3,7 @@
 // :946-989) and the full-spectrum variants (:678-755, :1112-1195).
 #pragma once
 #include "jt_fft1d.hpp"
+#include "jt_pair.hpp"
 
 namespace jt {
 
@@ -68,56 +69,6 @@ __global__ void real_to_complex(const T* __restrict__ x, cpx<T>* __restrict__ y,
                                 int64_t lines) {
     int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     for (; i < lines * n; i += (int64_t)gridDim.x * blockDim.x) y[i] = cpx<T>{x[i], T(0)};
-}
-
-// full spectrum (complex n) -> packed reals (n), both line stride n
-template <typename T>
-__global__ void pack_real(const cpx<T>* __restrict__ X, T* __restrict__ a, int64_t n, int64_t lines) {
-    int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    for (; i < lines * n; i += (int64_t)gridDim.x * blockDim.x) {
-        int64_t b = i / n, j = i % n;
-        const cpx<T>* Xb = X + b * n;
-        T v;
-        if (j == 0) v = Xb[0].x;
-        else if (j == 1) v = (n % 2 == 0) ? Xb[n / 2].x : Xb[(n - 1) / 2].y;
-        else if (j % 2 == 0) v = Xb[j / 2].x;
-        else v = Xb[j / 2].y;
-        a[i] = v;
-    }
-}
-
-// packed reals -> full Hermitian spectrum (complex n)
-template <typename T>
-__global__ void unpack_real(const T* __restrict__ a, cpx<T>* __restrict__ X, int64_t n, int64_t lines) {
-    int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    for (; i < lines * n; i += (int64_t)gridDim.x * blockDim.x) {
-        int64_t b = i / n, k = i % n;
-        const T* ab = a + b * n;
-        int64_t kk = k <= n / 2 ? k : n - k;
-        bool cj = k > n / 2;
-        T re, im;
-        if (kk == 0) {
-            re = ab[0];
-            im = 0;
-        } else if (n % 2 == 0 && kk == n / 2) {
-            re = ab[1];
-            im = 0;
-        } else if (n % 2 == 1 && kk == (n - 1) / 2) {
-            re = ab[2 * kk];
-            im = ab[1];
-        } else {
-            re = ab[2 * kk];
-            im = ab[2 * kk + 1];
-        }
-        X[i] = cpx<T>{re, cj ? -im : im};
-    }
-}
-
-// real parts of complex lines -> reals, times s
-template <typename T>
-__global__ void complex_real_part(const cpx<T>* __restrict__ X, T* __restrict__ a, int64_t count, T s) {
-    int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    for (; i < count; i += (int64_t)gridDim.x * blockDim.x) a[i] = X[i].x * s;
 }
 
 template <typename T>
@@ -191,18 +142,8 @@ void real_forward(const Real1D<T>& r, T* a, int64_t lines, cpx<T>* ws, hipStream
         }
         return;
     }
-    // odd n: full complex transform of the real input, then pack
-    cpx<T>* X = ws;
-    cpx<T>* ws2 = ws + lines * n;
-    { JT_PROF(st, "real_to_complex");
-    hipLaunchKernelGGL((real_to_complex<T>), ew_grid(lines * n), dim3(256), 0, st, a, X, n, lines);
-    }
-    JT_HIP(hipGetLastError());
-    c2c_contig<T, -1>(*r.full, X, X, lines, T(1), ws2, st);
-    { JT_PROF(st, "pack_real");
-    hipLaunchKernelGGL((pack_real<T>), ew_grid(lines * n), dim3(256), 0, st, X, a, n, lines);
-    }
-    JT_HIP(hipGetLastError());
+    // odd n
+    pair_lines<T, R2R_PACKED, true>(*r.full, a, nullptr, LineMap{lines, lines, n, 0, 1}, T(1), T(1), ws, st);
 }
 
 // Unscaled realInverse returns (n/2) x for powers of two and n x otherwise
@@ -235,19 +176,9 @@ void real_inverse(const Real1D<T>& r, T* a, int64_t lines, bool scale, cpx<T>* w
         }
         return;
     }
-    cpx<T>* X = ws;
-    cpx<T>* ws2 = ws + lines * n;
-    { JT_PROF(st, "unpack_real");
-    hipLaunchKernelGGL((unpack_real<T>), ew_grid(lines * n), dim3(256), 0, st, a, X, n, lines);
-    }
-    JT_HIP(hipGetLastError());
-    c2c_contig<T, 1>(*r.full, X, X, lines, T(1), ws2, st);
     // the backward sum is n x; unscaled non-power-of-two result is n x
-    { JT_PROF(st, "complex_real_part");
-    hipLaunchKernelGGL((complex_real_part<T>), ew_grid(lines * n), dim3(256), 0, st, X, a, lines * n,
-                       scale ? T(1.0 / (double)n) : T(1));
-    }
-    JT_HIP(hipGetLastError());
+    pair_lines<T, R2R_PACKED, false>(*r.full, a, nullptr, LineMap{lines, lines, n, 0, 1}, T(1),
+                                     scale ? T(1.0 / (double)n) : T(1), ws, st);
 }
 
 // realForwardFull / realInverseFull: complex transform of the real input

@@ -117,3 +117,47 @@ def test_bluestein(orc, n, prec):
     assert rel(a, orc.fftnd_complex([n, 6], x.astype(np.float64), -1)) <= tol(6 * n, prec)
     p.complexInverse(a, True)
     assert rel(a, x) <= 2 * tol(6 * n, prec)
+
+
+# odd lengths (one launch; Bluestein in one launch; several launches), 2, and
+# even ones whose half has a large prime factor
+PAIR = [2, 3, 9, 37, 74, 225, 999, 1021, 2047, 4095, 4103, 10158]
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("kind", ["dct", "dst", "dht"])
+@pytest.mark.parametrize("n", PAIR)
+def test_line_pairs(orc, kind, n, prec):
+    """Two real lines as one complex transform: contiguous and strided lines,
+    an odd number of them (the last pair has one line), both directions."""
+    for dims in ((3, n), (n, 5)):
+        x = orc.jrandom_doubles(n, n * dims[0 if dims[1] == n else 1]).astype(DT[prec])
+        p = R2R2[kind][prec == "f32"](*dims)
+        for fwd in (True, False):
+            a = x.copy()
+            if fwd:
+                p.forward(a, *([True] if kind != "dht" else []))
+            else:
+                p.inverse(a, True)
+            e = rel(a, orc.realnd(kind, list(dims), x.astype(np.float64), fwd, kind != "dht" or not fwd))
+            assert e <= tol(x.size, prec), (dims, fwd, e)
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("n", [3, 9, 37, 225, 1021, 4095, 4103, 33075])
+def test_odd_packed_batch(orc, n, prec):
+    """realForward / realInverse of odd lengths on a batch with a last single line."""
+    lines = 3
+    x = orc.jrandom_doubles(n, n * lines).astype(DT[prec])
+    p = jt.FFTBatch1D(n, lines, precision=prec)
+    a = x.copy()
+    p.realForward(a)
+    for b in range(lines):
+        s = slice(b * n, (b + 1) * n)
+        assert rel(a[s], orc.real_forward(n, x[s].astype(np.float64))) <= tol(n, prec), b
+    for scale in (True, False):
+        c = x.copy()
+        p.realInverse(c, scale)
+        for b in range(lines):
+            s = slice(b * n, (b + 1) * n)
+            assert rel(c[s], orc.real_inverse(n, x[s].astype(np.float64), scale)) <= 2 * tol(n, prec), (b, scale)
