@@ -326,7 +326,10 @@ def other_workload(args, torch, jt):
                 # (graph replays record no per-launch events: kernel time and
                 # roofline come from the direct launches)
                 rk = {k: v for k, v in prof.items() if k.startswith("ragged<")}
-                kern_ms = sum(v[1] for v in rk.values()) / sum(v[0] for v in rk.values()) if rk else None
+                # (a step is one launch, or one per pass)
+                if rk:
+                    rk = {next(iter(rk)): (K, sum(v[1] for v in rk.values()))}
+                kern_ms = next(iter(rk.values()))[1] / K if rk else None
                 rf = roofline_from_profile(rk, alg_override=byt) if rk else None
                 if rf:
                     rf.pop("kernels")
@@ -335,7 +338,7 @@ def other_workload(args, torch, jt):
                             "schedule": plan.describe(), "kernel_ms": kern_ms, "roofline": rf}
                 del bufs, base, plan
         out.update({"config": "ragged batch of 20000 1D complex transforms, n log-uniform in [16, 65536] "
-                              "(70% 2^a3^b5^c, 25% 2^k, 5% primes), one persistent launch",
+                              "(70% 2^a3^b5^c, 25% 2^k, 5% primes), one plan",
                     "total_points": int(lens.sum()), "flops": flops, "results": res})
         return out
 
@@ -403,14 +406,18 @@ def _benched_launches(launches):
     """The launches of the schedule that was timed.  A ragged batch's label
     carries its schedule, and its family also holds the autotuner's trial
     launches: keep those of the label launched most often (the timed steps
-    repeat the tuned schedule).  Other families are returned whole."""
-    counts = {}
-    for _, _, lab in launches:
-        counts[lab] = counts.get(lab, 0) + 1
+    repeat the tuned schedule), one entry per execution where that is one
+    launch per pass.  Other families are returned whole."""
     if not launches or not launches[0][2].startswith("ragged<"):
         return launches
+    sched = [re.sub(r",pass=[^>]*", "", x[2]) for x in launches]
+    counts = {}
+    for lab in sched:
+        counts[lab] = counts.get(lab, 0) + 1
     best = max(counts, key=counts.get)
-    return [x for x in launches if x[2] == best]
+    mine = [x for x, lab in zip(launches, sched) if lab == best]
+    passes = len({x[2] for x in mine})
+    return [(sum(x[0] for x in mine[i:i + passes]), mine[i][1], best) for i in range(0, len(mine), passes)]
 
 
 MIN_LISTED_BYTES = 32 << 20

@@ -116,7 +116,7 @@ int jt_plan_create_fft1d_batch(jt_plan** out, int precision, int64_t n, int64_t 
 
 /* `count` independent 1D complex transforms of the given lengths, stored
  * back to back (transform i starts at element 2*sum_{j<i} lengths[j]), run in
- * one persistent launch (JT_COMPLEX_FORWARD / JT_COMPLEX_INVERSE, scale = 1/n
+ * one persistent launch or one launch per pass (JT_COMPLEX_FORWARD / JT_COMPLEX_INVERSE, scale = 1/n
  * per transform).  No counterpart in the reference, whose callers build one
  * DoubleFFT_1D per length (fft/DoubleFFT_1D.java:117) and call it per
  * transform. */

@@ -372,8 +372,8 @@ class FFTBatch1D(_FFTMethods):
 
 class RaggedBatch1D(_Plan):
     """Many 1D complex transforms of unequal lengths stored back to back, run
-    in one persistent launch (no reference counterpart: it replaces one
-    DoubleFFT_1D per length).  graph=True replays a captured hipGraph."""
+    in one persistent launch or one launch per pass (no reference counterpart:
+    it replaces one DoubleFFT_1D per length).  graph=True replays a captured hipGraph."""
 
     def __init__(self, lengths, precision: str = "f64", graph: bool = False, autotune: bool = False):
         self._precision = JT_F64 if precision in ("f64", "double") else JT_F32

@@ -640,6 +640,30 @@ bool dispatch_tpl(int64_t n, IO io, const cpx<T>* tw, hipStream_t st, bool mf = 
     return dispatch_tpl_n<T, DIR, COL>(n, io, tw, st);
 }
 
+// Threads that W lines of the plan need (see gen_butterflies).
+inline int gen_threads(const GenPlan& g, int W) {
+    int nt = 64;
+    for (int s = 0; s < g.nst; s++) {
+        const int per = gen_butterflies(g.st[s].radix);
+        nt = std::max(nt, (g.st[s].m * W + per - 1) / per);
+    }
+    return (nt + 63) / 64 * 64;
+}
+// LDS elements from line to line: the lines fall into disjoint bank groups
+// (as in LdsGeom).
+inline int gen_pitch(int n, int W) {
+    const int p = n + (n >> 5) + 1;
+    const int off = 16 / W > 0 ? 16 / W : 1;
+    return W == 1 ? p : p + (off - p % 32 + 64) % 32;
+}
+inline void gen_set_shape(GenPlan& g, int W, bool col) {
+    g.W = W;
+    g.lgW = 0;
+    while ((1 << g.lgW) < W) g.lgW++;
+    g.col = col ? 1 : 0;
+    g.pitch = gen_pitch(g.n, W);
+}
+
 // Launch shape of the runtime-radix kernel: W lines and NT threads per
 // workgroup.  eb: bytes of one element of a line in memory.  The lines lie
 // where these were fastest (us for a forward and a backward pass):
@@ -661,22 +685,11 @@ struct GenShape {
 template <typename T>
 GenShape gen_shape(GenPlan& g, int64_t nlines, bool col, int eb, bool hooks) {
     const int n = g.n;
-    auto pitch_of = [&](int W) {
-        // lines fall into disjoint bank groups (as LdsGeom)
-        const int p = n + (n >> 5) + 1;
-        const int off = 16 / W > 0 ? 16 / W : 1;
-        return W == 1 ? p : p + (off - p % 32 + 64) % 32;
-    };
     auto threads = [&](int W) {
-        int nt = 64;
-        for (int s = 0; s < g.nst; s++) {
-            const int per = gen_butterflies(g.st[s].radix);
-            nt = std::max(nt, (g.st[s].m * W + per - 1) / per);
-        }
-        if (!hooks) nt = std::max(nt, std::min(1024, n * W / 8));
-        return (nt + 63) / 64 * 64;
+        const int nt = gen_threads(g, W);
+        return hooks ? nt : std::max(nt, (std::min(1024, n * W / 8) + 63) / 64 * 64);
     };
-    auto bytes = [&](int W) { return 2 * (size_t)W * pitch_of(W) * sizeof(T); };
+    auto bytes = [&](int W) { return 2 * (size_t)W * gen_pitch(n, W) * sizeof(T); };
     auto fits = [&](int W, size_t lds) { return W <= 64 && threads(W) <= 1024 && bytes(W) <= lds; };
     auto groups = [&](int W) { return (nlines + W - 1) / W; };
     int W = 1;
@@ -696,11 +709,7 @@ GenShape gen_shape(GenPlan& g, int64_t nlines, bool col, int eb, bool hooks) {
     const int most = std::min(1024, n * W / (hooks ? 2 : 4));
     while (2 * nt <= most && groups(W) * nt < (int64_t(1) << 18)) nt *= 2;
     if (!fits(W, 160 * 1024)) throw JtError(ST_UNSUPPORTED, "internal: length beyond the runtime-radix kernel");
-    g.W = W;
-    g.lgW = 0;
-    while ((1 << g.lgW) < W) g.lgW++;
-    g.col = col ? 1 : 0;
-    g.pitch = pitch_of(W);
+    gen_set_shape(g, W, col);
     return GenShape{W, nt, bytes(W)};
 }
 

@@ -143,7 +143,7 @@ constexpr int gen_butterflies(int R) { return GEN_PTS / R > 0 ? GEN_PTS / R : 1;
 // LDS.  TOG: the outputs go through io.store; else to LDS, in place (all
 // inputs are in registers before the barrier that precedes the first write;
 // the host sizes NT so that gen_butterflies(R) per thread cover the stage).
-// SPEC: each output k is multiplied by io.spec(line, k) and conjugated (the
+// SPEC: each output k is multiplied by io.spec(at, k) and conjugated (the
 // middle of a convolution).
 template <int R, int DIR, bool FROMG, bool TOG, bool SPEC, typename T, class IO>
 __device__ __forceinline__ void gen_stage(const IO& io, GenStage S, int W, int lgW, int pitch, bool col,
@@ -205,7 +205,7 @@ __device__ __forceinline__ void gen_stage(const IO& io, GenStage S, int W, int l
                     // a store that loads factors of its own: a few at a time,
                     // or their registers spill
                     if constexpr (IO::store_loads)
-                        if (sizeof(T) == 8 || r % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+                        if (r % (sizeof(T) == 8 ? 2 : 4) == 1) __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
                 T* lr = re + ww[b] * pitch;
@@ -215,7 +215,7 @@ __device__ __forceinline__ void gen_stage(const IO& io, GenStage S, int W, int l
                 for (int r = 0; r < R; r++) {
                     const int k = gpos(d + r * ns);
                     if constexpr (SPEC) {
-                        const cpx<T> p = cmul(v[b][r], io.spec(line0 + ww[b], d, r * ns));
+                        const cpx<T> p = cmul(v[b][r], io.spec(io.base(line0 + ww[b]), d, r * ns));
                         v[b][r] = cpx<T>{p.x, -p.y};
                         if (sizeof(T) == 8 || r % 2 == 1) __builtin_amdgcn_sched_barrier(0);
                     }
@@ -268,32 +268,41 @@ __device__ __forceinline__ int64_t xcd_group(int64_t bid, int64_t ngroups) {
     return (bid % nx) * per + bid / nx;
 }
 
-// IO contract as for stockham_kernel, except that loads and stores name the
-// element as j + rm with rm uniform over the workgroup; pre/post hooks work on
-// one line with the threads (t, nt) of that line and address LDS through
-// gpos(k).  A policy with conv = true runs the transform twice with the
-// spectrum product between: out = DFT(conj(spec * DFT(in))), i.e. a cyclic
-// convolution up to a conjugation that its store undoes, in one LDS residency
-// (nst >= 2).
-template <typename T, int DIR, class IO>
-__global__ void __launch_bounds__(1024) generic_kernel(IO io, const cpx<T>* __restrict__ tw, GenPlan P) {
+// Read-only tables of a plan are read through the constant address space: the
+// compiler then knows that the kernel's stores never change them, so their
+// loads are hoisted and batched across stores, and loads at a wave-uniform
+// address become scalar loads.
+template <class X>
+using ro_ptr = const __attribute__((address_space(4))) X*;
+template <class X>
+__device__ __forceinline__ ro_ptr<X> ro(const X* p) { return (ro_ptr<X>)p; }
+__device__ __forceinline__ GenStage stage_of(const GenPlan& P, int s) { return P.st[s]; }
+__device__ __forceinline__ GenStage stage_of(ro_ptr<GenPlan> P, int s) {
+    return GenStage{P->st[s].radix, P->st[s].m, P->st[s].ns, P->st[s].twoff, P->st[s].rm, P->st[s].rns};
+}
+
+// The lines line0 .. line0+nl-1 (nl <= W) through all stages.  IO contract as
+// for stockham_kernel, except that loads and stores name the element as j + rm
+// with rm uniform over the workgroup; pre/post hooks work on one line with the
+// threads (t, nt) of that line and address LDS through gpos(k).  A policy with
+// conv = true runs the transform twice with the spectrum product between:
+// out = DFT(conj(spec * DFT(in))), i.e. a cyclic convolution up to a
+// conjugation that its store undoes, in one LDS residency (nst >= 2).
+// `stages` is the plan's stage list, as a kernel argument or in memory.
+template <typename T, int DIR, class IO, class Stages>
+__device__ __forceinline__ void gen_lines(const IO& io, const cpx<T>* __restrict__ tw, const Stages& stages, int nst,
+                                          int n, int W, int lgW, int pitch, bool col, int64_t line0, int nl) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    const int W = P.W;
     T* re = reinterpret_cast<T*>(smem_raw);
-    T* im = re + W * P.pitch;
+    T* im = re + W * pitch;
     const int tid = threadIdx.x;
-    const int64_t ngroups = (io.nlines + W - 1) / W;
-    const int64_t bid = blockIdx.x + (int64_t)blockIdx.y * gridDim.x;
-    if (bid >= ngroups) return;  // whole workgroup exits together
-    const int64_t line0 = (io.xcd ? xcd_group(bid, ngroups) : bid) * W;
-    const int nl = (int)(io.nlines - line0 < W ? io.nlines - line0 : W);
     // the hooks' view: line hw, thread ht of hn
     int hw = 0, ht = tid, hn = blockDim.x;
     if constexpr (IO::pre_lds || IO::post_lds) {
         hn = blockDim.x / W;
-        if (P.col) {
+        if (col) {
             hw = tid & (W - 1);
-            ht = tid >> P.lgW;
+            ht = tid >> lgW;
         } else if (W > 1) {
             hw = tid / hn;
             ht = tid - hw * hn;
@@ -302,43 +311,54 @@ __global__ void __launch_bounds__(1024) generic_kernel(IO io, const cpx<T>* __re
     int s = 0;
     if constexpr (IO::pre_lds) {
         if (hw < nl)
-            io.template pre<0, 0>(line0 + hw, io.base(line0 + hw), re + hw * P.pitch, im + hw * P.pitch, ht, hn);
-    } else if (P.nst > 0) {
-        gen_stage_rt<DIR, true, false>(io, P.st[0], W, P.lgW, P.pitch, P.col, tw, re, im, line0, nl, tid);
+            io.template pre<0, 0>(line0 + hw, io.base(line0 + hw), re + hw * pitch, im + hw * pitch, ht, hn);
+    } else if (nst > 0) {
+        gen_stage_rt<DIR, true, false>(io, stage_of(stages, 0), W, lgW, pitch, col, tw, re, im, line0, nl, tid);
         s = 1;
     } else if (tid < nl) {  // n == 1
         const cpx<T> x = io.load(io.base(line0 + tid), 0, 0);
-        re[tid * P.pitch] = x.x;
-        im[tid * P.pitch] = x.y;
+        re[tid * pitch] = x.x;
+        im[tid * pitch] = x.y;
     }
     // (one loop over both transforms of a convolution: with two, the compiler
     // keeps a copy of the stage list in scratch)
-    const int all = IO::conv ? 2 * P.nst : P.nst;
+    const int all = IO::conv ? 2 * nst : nst;
     const int inner = IO::post_lds ? all : all - 1;
     for (; s < inner; s++) {
-        const GenStage S = P.st[IO::conv && s >= P.nst ? s - P.nst : s];
+        const GenStage S = stage_of(stages, IO::conv && s >= nst ? s - nst : s);
         __syncthreads();
         if constexpr (IO::conv) {
-            if (s == P.nst - 1) {
-                gen_stage_rt<DIR, false, false, true>(io, S, W, P.lgW, P.pitch, P.col, tw, re, im, line0, nl, tid);
+            if (s == nst - 1) {
+                gen_stage_rt<DIR, false, false, true>(io, S, W, lgW, pitch, col, tw, re, im, line0, nl, tid);
                 continue;
             }
         }
-        gen_stage_rt<DIR, false, false>(io, S, W, P.lgW, P.pitch, P.col, tw, re, im, line0, nl, tid);
+        gen_stage_rt<DIR, false, false>(io, S, W, lgW, pitch, col, tw, re, im, line0, nl, tid);
     }
     __syncthreads();
     if constexpr (IO::post_lds) {
         if (hw < nl)
-            io.template post<0, 0>(line0 + hw, io.base(line0 + hw), re + hw * P.pitch, im + hw * P.pitch, ht, hn);
+            io.template post<0, 0>(line0 + hw, io.base(line0 + hw), re + hw * pitch, im + hw * pitch, ht, hn);
     } else if (s < all) {
-        gen_stage_rt<DIR, false, true>(io, P.st[P.nst - 1], W, P.lgW, P.pitch, P.col, tw, re, im, line0, nl, tid);
+        gen_stage_rt<DIR, false, true>(io, stage_of(stages, nst - 1), W, lgW, pitch, col, tw, re, im, line0, nl, tid);
     } else {
         // one stage at most: the results are in LDS
-        for (int idx = tid; idx < nl * P.n; idx += blockDim.x) {
-            const int w = P.col ? idx % nl : idx / P.n, k = P.col ? idx / nl : idx % P.n;
-            io.store(io.base(line0 + w), k, 0, cpx<T>{re[w * P.pitch + gpos(k)], im[w * P.pitch + gpos(k)]});
+        for (int idx = tid; idx < nl * n; idx += blockDim.x) {
+            const int w = col ? idx % nl : idx / n, k = col ? idx / nl : idx % n;
+            io.store(io.base(line0 + w), k, 0, cpx<T>{re[w * pitch + gpos(k)], im[w * pitch + gpos(k)]});
         }
     }
+}
+
+template <typename T, int DIR, class IO>
+__global__ void __launch_bounds__(1024) generic_kernel(IO io, const cpx<T>* __restrict__ tw, GenPlan P) {
+    const int W = P.W;
+    const int64_t ngroups = (io.nlines + W - 1) / W;
+    const int64_t bid = blockIdx.x + (int64_t)blockIdx.y * gridDim.x;
+    if (bid >= ngroups) return;  // whole workgroup exits together
+    const int64_t line0 = (io.xcd ? xcd_group(bid, ngroups) : bid) * W;
+    const int nl = (int)(io.nlines - line0 < W ? io.nlines - line0 : W);
+    gen_lines<T, DIR>(io, tw, P, P.nst, P.n, W, P.lgW, P.pitch, P.col, line0, nl);
 }
 
 }  // namespace jt

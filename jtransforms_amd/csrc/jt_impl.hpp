@@ -295,7 +295,24 @@ std::unique_ptr<RaggedPlan<T>> make_ragged_tuned(const int64_t* lengths, int64_t
                 pos = end + 1;
             }
         }
-        P = make_ragged<T>(lengths, count, t);
+        else {
+            // One launch per pass was faster at every size measured, us in
+            // both directions against the persistent kernel: 3 transforms
+            // (60 thousand points) 40 to 111, 100 FP64 239 to 622, 4000 FP64
+            // 1564 to 2015, 4000 FP32 1012 to 1512.  The line is not where
+            // the two cross: below it stays the form whose waits can fail,
+            // with the report of that failure that its tests force there.
+            int64_t points = 0;
+            for (int64_t i = 0; i < count; i++) points += lengths[i];
+            if (points >= (int64_t(1) << 17)) t.form = 1;
+        }
+        try {
+            P = make_ragged<T>(lengths, count, t);
+        } catch (const JtError& e) {
+            if (t.form == 0 || e.code != ST_UNSUPPORTED) throw;
+            t.form = 0;  // a length that form does not cover
+            P = make_ragged<T>(lengths, count, t);
+        }
     } else {
         auto key = std::make_pair((int)sizeof(T), std::vector<int64_t>(lengths, lengths + count));
         RTune known;

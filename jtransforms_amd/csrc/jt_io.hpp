@@ -246,7 +246,7 @@ struct IOBlueL {
         else if constexpr (PASS == 2) return ws[(a.w + a.q * n2 + k) + rm];
         else return ws[(a.w + a.q + k * n2) + rm * n2];
     }
-    __device__ __forceinline__ cpx<T> spec(int64_t l, int k, int rm) const { return c.spec(l % n1 * n2 + k + rm); }
+    __device__ __forceinline__ cpx<T> spec(At a, int k, int rm) const { return c.spec(a.q * n2 + k + rm); }
     __device__ __forceinline__ void store(At a, int k, int rm, cpx<T> v) const {
         if constexpr (PASS == 1) {
             ws[(a.w + a.q + k * n2) + rm * n2] = cmul(v, tw2<-1>(hi, lo, a.q * k + a.q * rm));

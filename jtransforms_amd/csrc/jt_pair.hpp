@@ -90,7 +90,7 @@ struct IOPair {
     }
     __device__ cpx<T> load(At, int, int) const { return cpx<T>{T(0), T(0)}; }
     __device__ void store(At, int, int, cpx<T>) const {}
-    __device__ __forceinline__ cpx<T> spec(int64_t, int k, int rm) const { return c.spec(k + rm); }
+    __device__ __forceinline__ cpx<T> spec(At, int k, int rm) const { return c.spec(k + rm); }
 
     // inverse: z_k = n (v_a + i v_b) back into the lines
     __device__ __forceinline__ void join(At at, I k, cpx<T> z) const {

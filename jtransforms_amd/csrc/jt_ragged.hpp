@@ -32,6 +32,7 @@
 
 #include "jt_generic.hpp"
 #include "jt_fft1d.hpp"
+#include "jt_ragpass.hpp"
 
 namespace jt {
 
@@ -107,14 +108,18 @@ struct RArgs {
 //          follow the phase before it, so that it reads the workspace
 //          written shortly before, from the last-level cache, rather than
 //          from HBM, and its wait for that phase has normally ended
+//   form   0: this persistent kernel; 1: one launch per pass (jt_ragpass.hpp),
+//          which the other knobs do not apply to
 struct RTune {
     int wgs = 2, nt = 0, tplx = 0, chunk = 4, order = 0, lag = 0;  // nt 0: smallest that fits
+    int form = 0;
     std::string str() const {
         return "wgs=" + std::to_string(wgs) + ",nt=" + std::to_string(nt) + ",tplx=" + std::to_string(tplx) +
-               ",chunk=" + std::to_string(chunk) + ",order=" + std::to_string(order) + ",lag=" + std::to_string(lag);
+               ",chunk=" + std::to_string(chunk) + ",order=" + std::to_string(order) + ",lag=" + std::to_string(lag) + (form ? ",form=launches" : "");
     }
     bool operator==(const RTune& o) const {
-        return wgs == o.wgs && nt == o.nt && tplx == o.tplx && chunk == o.chunk && order == o.order && lag == o.lag;
+        return wgs == o.wgs && nt == o.nt && tplx == o.tplx && chunk == o.chunk && order == o.order && lag == o.lag &&
+               form == o.form;
     }
 };
 
@@ -126,14 +131,6 @@ struct RTune {
 // compiler cannot tell, so it is moved to a scalar register explicitly.
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// Read-only tables of the plan (descriptors, items, offsets, twiddles) are
-// read through the constant address space: the compiler then knows that the
-// kernel's stores never change them, so their loads are hoisted and batched
-// across stores, and loads at a wave-uniform address become scalar loads.
-template <class X>
-using ro_ptr = const __attribute__((address_space(4))) X*;
-template <class X>
-__device__ __forceinline__ ro_ptr<X> ro(const X* p) { return (ro_ptr<X>)p; }
 template <typename T>
 __device__ __forceinline__ cpx<T> rd(ro_ptr<cpx<T>> p, int64_t i) { return cpx<T>{p[i].x, p[i].y}; }
 
@@ -559,6 +556,7 @@ struct RaggedPlan {
     size_t shm = 0;
     int np = 0;
     RTune tune;
+    std::unique_ptr<RaggedPasses<T>> passes;  // form 1
     // hipGraph cache: one executable graph per (data, stream, dir, scale)
     struct GKey {
         void* data;
@@ -638,6 +636,36 @@ std::unique_ptr<RaggedPlan<T>> make_ragged(const int64_t* lengths, int64_t count
         tune.lag < 0 || tune.lag > (1 << 20))
         throw JtError(ST_BAD_ARG, "ragged schedule out of range (wgs 1..8, nt 0/256/512/1024, tplx 0..4, "
                                   "chunk 1..1024, order 0/1, lag 0..2^20): " + tune.str());
+    // (chirp, spectrum) of a Bluestein length
+    auto blue_tables = [&](int64_t n, int64_t m, std::vector<cpx<double>>& ch, std::vector<cpx<double>>& bs) {
+        if (spec_cache && spec_cache->count(n)) {
+            ch = (*spec_cache)[n].first;
+            bs = (*spec_cache)[n].second;
+            return;
+        }
+        // chirp exp(i pi (j^2 mod 2n)/n) by the integer recurrence
+        ch.resize(n);
+        const long double PI = 3.141592653589793238462643383279502884L;
+        int64_t k = 0;
+        for (int64_t j = 0; j < n; j++) {
+            if (j) {
+                k += 2 * j - 1;
+                if (k >= 2 * n) k -= 2 * n;
+            }
+            long double ang = PI * (long double)k / (long double)n;
+            ch[j] = cpx<double>{(double)cosl(ang), (double)sinl(ang)};
+        }
+        bs = bluestein_spectrum(n, m, ch);
+        if (spec_cache) (*spec_cache)[n] = std::make_pair(ch, bs);
+    };
+    if (tune.form == 1) {
+        P->passes = make_passes<T>(lengths, count, blue_tables);
+        if (!P->passes) throw JtError(ST_UNSUPPORTED, "length too large for one launch per pass");
+        for (int64_t i = 0; i < count; i++) P->total += lengths[i];
+        P->d_err.alloc(sizeof(int));
+        JT_HIP(hipMemset(P->d_err.p, 0, sizeof(int)));
+        return P;
+    }
     std::vector<RLen> lens;
     std::vector<cpx<T>> tab;
     int max_tpl = 1;                     // largest threads-per-line requirement
@@ -711,25 +739,7 @@ std::unique_ptr<RaggedPlan<T>> make_ragged(const int64_t* lengths, int64_t count
             L.m = (int)m;
             L.kind = m <= lim ? RK_BLUE_S : RK_BLUE_L;
             std::vector<cpx<double>> ch, bs;
-            if (spec_cache && spec_cache->count(n)) {
-                ch = (*spec_cache)[n].first;
-                bs = (*spec_cache)[n].second;
-            } else {
-                // chirp exp(i pi (j^2 mod 2n)/n) by the integer recurrence
-                ch.resize(n);
-                const long double PI = 3.141592653589793238462643383279502884L;
-                int64_t k = 0;
-                for (int64_t j = 0; j < n; j++) {
-                    if (j) {
-                        k += 2 * j - 1;
-                        if (k >= 2 * n) k -= 2 * n;
-                    }
-                    long double ang = PI * (long double)k / (long double)n;
-                    ch[j] = cpx<double>{(double)cosl(ang), (double)sinl(ang)};
-                }
-                bs = bluestein_spectrum(n, m, ch);
-                if (spec_cache) (*spec_cache)[n] = std::make_pair(ch, bs);
-            }
+            blue_tables(n, m, ch, bs);
             L.choff = (int64_t)tab.size();
             for (auto& c : ch) tab.push_back(cpx<T>{(T)c.x, (T)c.y});
             L.bsoff = (int64_t)tab.size();
@@ -971,6 +981,12 @@ RArgs<T> ragged_args(RaggedPlan<T>& P, cpx<T>* data, int dir, bool scaled) {
 
 template <typename T>
 void ragged_launch(RaggedPlan<T>& P, cpx<T>* data, int dir, bool scaled, hipStream_t st) {
+    if (P.passes) {
+        passes_launch<T>(*P.passes, data, dir, scaled,
+                         std::string("ragged<") + (sizeof(T) == 8 ? "f64" : "f32") + ",transforms=" +
+                             std::to_string(P.ntr) + ",points=" + std::to_string(P.total) + "," + P.tune.str(), st);
+        return;
+    }
     RArgs<T> a = ragged_args(P, data, dir, scaled);
     {
         JT_PROF(st, "ragged_reset");
@@ -1112,6 +1128,9 @@ std::unique_ptr<RaggedPlan<T>> ragged_autotune(const int64_t* lengths, int64_t c
                 consider(t);
             }
         }
+        RTune t = best->tune;
+        t.form = 1;
+        consider(t);
     } catch (...) {
         cleanup();
         throw;

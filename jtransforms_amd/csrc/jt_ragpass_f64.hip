@@ -1,0 +1,6 @@
+// FP64 ragged batches, one launch per pass.
+#include "jt_ragpass.hpp"
+
+namespace jt {
+JT_RAGPASS_INST(, double)
+}  // namespace jt
