@@ -124,7 +124,7 @@ int create(jt_plan** out, int family, int precision, int ndim, const int64_t* di
 // Does `op` touch the plan's device buffers (beyond the tables, which are
 // read-only)?  Then calls on different streams are ordered (see jt_plan).
 bool touches_plan_buffers(const jt_plan* p, int op, bool staged) {
-    return staged || p->family == FAM_RAGGED || p->op_ws[op] > 0;
+    return staged || p->family == FAM_RAGGED || p->op_ws_used[op];
 }
 
 // The plan's workspace of `op`, and its staging area after it.

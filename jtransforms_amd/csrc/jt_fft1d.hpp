@@ -321,6 +321,8 @@ struct Fft1D {
     bool single() const { return kind == K_TPL || kind == K_GEN; }
     // Bluestein in one launch, on lines of any stride
     bool blue_single() const { return kind == K_BLUE && pm->kind == K_GEN; }
+    // one launch without workspace, on lines of any stride
+    bool one_launch() const { return single() || blue_single(); }
     // workspace (complex elements) for `lines` contiguous lines
     int64_t workspace(int64_t lines) const {
         if (kind == K_FOUR) return lines * n + (p2->single() ? 0 : p2->workspace(lines * n1));
@@ -879,7 +881,7 @@ void c2c_contig(const Fft1D<T>& p, const cpx<T>* in, cpx<T>* out, int64_t lines,
         if (!p.p1->single()) throw JtError(ST_UNSUPPORTED, "four-step column plan must be single-kernel");
         const bool two = p.p2->single();
         IOFourA<T, DIR> a{in, ws, p.hi.template as<cpx<T>>(), p.lo.template as<cpx<T>>(), lines * p.n2,
-                          p.n, p.n1, p.n2, two ? p.n1 : 1, two ? 1 : p.n2, true};
+                          p.n, p.n1, p.n2, two ? p.n1 : 1, two ? 1 : p.n2, true, LineDiv(lines * p.n2, p.n2)};
         run_single<T, DIR, true>(*p.p1, a, st);
         if (two) {
             // pass A left the transpose: the n2-point rows are columns of an
@@ -909,9 +911,9 @@ void c2c_contig(const Fft1D<T>& p, const cpx<T>* in, cpx<T>* out, int64_t lines,
         const Chirp<T> c{p.chirp.template as<cpx<T>>(), p.bspec.template as<cpx<T>>(), p.n, T(DIR)};
         const cpx<T>* hi = f.hi.template as<cpx<T>>();
         const cpx<T>* lo = f.lo.template as<cpx<T>>();
-        go_gen<T, -1>(*p.pa, IOBlueL<T, 1>{in, out, ws, c, hi, lo, lines * f.n2, f.n1, f.n2, scale, true}, true, st);
-        go_gen<T, -1>(*p.pb, IOBlueL<T, 2>{in, out, ws, c, hi, lo, lines * f.n1, f.n1, f.n2, scale, false}, false, st);
-        go_gen<T, 1>(*p.pa, IOBlueL<T, 3>{in, out, ws, c, hi, lo, lines * f.n2, f.n1, f.n2, scale, true}, true, st);
+        go_gen<T, -1>(*p.pa, IOBlueL<T, 1>{in, out, ws, c, hi, lo, lines * f.n2, f.n1, f.n2, scale, true, LineDiv(lines * f.n2, f.n2)}, true, st);
+        go_gen<T, -1>(*p.pb, IOBlueL<T, 2>{in, out, ws, c, hi, lo, lines * f.n1, f.n1, f.n2, scale, false, LineDiv(lines * f.n1, f.n1)}, false, st);
+        go_gen<T, 1>(*p.pa, IOBlueL<T, 3>{in, out, ws, c, hi, lo, lines * f.n2, f.n1, f.n2, scale, true, LineDiv(lines * f.n2, f.n2)}, true, st);
         return;
     }
     // a convolution beyond two levels

@@ -9,18 +9,28 @@ namespace jt {
 
 __device__ __forceinline__ int lpos(int k) { return k + (k >> 5); }
 
+// l / n0 for 0 <= l < nlines as a multiply by mag = floor(2^64 / n0) + 1
+// (exact while l * n0 < 2^64); mag 0 where the quotient is always 0.  Straight
+// code: a 64-bit division takes over a hundred instructions, and a branch
+// around it puts the kernel arguments behind it a second, late load.
+struct LineDiv {
+    int64_t n0;
+    uint64_t mag;
+    __host__ __device__ LineDiv(int64_t nlines, int64_t d) : n0(d), mag(nlines <= d ? 0 : ~uint64_t(0) / d + 1) {}
+    __device__ __forceinline__ int64_t operator()(int64_t l) const { return (int64_t)__umul64hi((uint64_t)l, mag); }
+};
+
 // Lines l in [0, nlines) start at (l % n0)*s0 + (l / n0)*s1 (complex units);
-// element k of a line sits es further per step.
+// element k of a line sits es further per step.  (n0 = 1 is the same as
+// n0 = nlines with s0 = s1.)
 struct LineMap {
-    int64_t nlines, n0, s0, s1, es;
+    int64_t nlines, s0, s1, es;
+    LineDiv div;
+    __host__ __device__ LineMap(int64_t nl, int64_t n0, int64_t s0_, int64_t s1_, int64_t es_)
+        : nlines(nl), s0(n0 == 1 ? s1_ : s0_), s1(s1_), es(es_), div(nl, n0 == 1 ? nl : n0) {}
     __device__ __forceinline__ int64_t base(int64_t l) const {
-        // (a 64-bit division by a run-time value takes over a hundred instructions)
-        if (nlines <= n0) return l * s0;
-        if (((uint64_t)nlines | (uint64_t)n0) >> 32 == 0) {
-            const uint32_t q = (uint32_t)l / (uint32_t)n0;
-            return (int64_t)((uint32_t)l - q * (uint32_t)n0) * s0 + (int64_t)q * s1;
-        }
-        return (l % n0) * s0 + (l / n0) * s1;
+        const int64_t q = div(l);
+        return (l - q * div.n0) * s0 + q * s1;
     }
 };
 
@@ -136,12 +146,12 @@ struct IOFourA {
     const cpx<T>* lo;
     int64_t nlines, n, n1, n2, oj, ok;
     bool xcd;
+    LineDiv div;  // by n2
     struct At {
         int64_t i, o, j2;
     };
     __device__ __forceinline__ At base(int64_t l) const {
-        if (nlines == n2) return At{l, l * oj, l};  // one transform
-        const int64_t b = l / n2, j2 = l - b * n2;
+        const int64_t b = div(l), j2 = l - b * n2;
         return At{b * n + j2, b * n + j2 * oj, j2};
     }
     __device__ __forceinline__ cpx<T> load(At a, int k, int rm) const { return in[(a.i + k * n2) + rm * n2]; }
@@ -209,6 +219,42 @@ struct IOBlue {
     }
 };
 
+// Contiguous lines of n reals in, n complex points out (realForwardFull and
+// realInverseFull), per line or, with the chirp, as a Bluestein transform.
+template <typename T>
+struct IORealRows {
+    static constexpr bool pre_lds = false, post_lds = false, store_loads = false, conv = false;
+    static const char* tag() { return "real rows"; }
+    std::string desc() const { return ",n=" + std::to_string(n); }
+    const T* in;
+    cpx<T>* out;
+    int64_t n, nlines;
+    T scale;
+    bool xcd;
+    __device__ __forceinline__ int64_t base(int64_t l) const { return l * n; }
+    __device__ __forceinline__ cpx<T> load(int64_t b, int k, int rm) const { return cpx<T>{in[b + k + rm], T(0)}; }
+    __device__ __forceinline__ void store(int64_t b, int k, int rm, cpx<T> v) const {
+        out[b + k + rm] = cpx<T>{v.x * scale, v.y * scale};
+    }
+    template <int CN, int CTL>
+    __device__ void pre(int64_t, int64_t, T*, T*, int, int) const {}
+    template <int CN, int CTL>
+    __device__ void post(int64_t, int64_t, const T*, const T*, int, int) const {}
+};
+template <typename T>
+struct IORealRowsBlue : IORealRows<T> {
+    static constexpr bool store_loads = true, conv = true;
+    Chirp<T> c;
+    __device__ __forceinline__ cpx<T> load(int64_t b, int k, int rm) const {
+        return c.premul(k + rm, [&](int64_t kk) { return cpx<T>{this->in[b + kk], T(0)}; });
+    }
+    __device__ __forceinline__ cpx<T> spec(int64_t, int k, int rm) const { return c.spec(k + rm); }
+    __device__ __forceinline__ void store(int64_t b, int k, int rm, cpx<T> v) const {
+        const int64_t kk = k + rm;
+        if (kk < c.n) this->out[b + kk] = c.postmul(kk, cpx<T>{v.x, -v.y}, this->scale);
+    }
+};
+
 // Longer convolutions, m = n1*n2, in three passes over an n1 x n2 matrix in
 // the workspace: the premultiplied, zero-padded columns (FFT over n1, times
 // exp(-2 pi i j2 k1/m)); the rows (FFT over n2, spectrum product, inverse FFT,
@@ -230,15 +276,14 @@ struct IOBlueL {
     int64_t nlines, n1, n2;
     T scale;
     bool xcd;
+    LineDiv div;  // by the lines of a transform
     struct At {
         int64_t x, w;  // offsets of the transform's data and matrix
         int64_t q;     // column j2 (passes 1, 3) or row k1 (pass 2)
     };
     __device__ __forceinline__ At base(int64_t l) const {
-        const int64_t per = PASS == 2 ? n1 : n2;
-        if (nlines == per) return At{0, 0, l};  // one transform
-        const int64_t b = l / per;
-        return At{b * c.n, b * n1 * n2, l - b * per};
+        const int64_t b = div(l);
+        return At{b * c.n, b * n1 * n2, l - b * div.n0};
     }
     __device__ __forceinline__ cpx<T> load(At a, int k, int rm) const {
         if constexpr (PASS == 1)

@@ -25,6 +25,13 @@ __global__ void scatter_lines(const cpx<T>* __restrict__ y, cpx<T>* __restrict__
     }
 }
 
+// One axis pass over lines lm from `in` to `out`, for a plan of one launch.
+template <typename T, int DIR>
+void axis_one(const Fft1D<T>& p, const cpx<T>* in, cpx<T>* out, LineMap lm, T scale, hipStream_t st) {
+    if (p.single()) c2c_mapped<T, DIR>(p, in, out, lm, scale, st);
+    else blue_mapped<T, DIR>(p, in, out, lm, scale, st);
+}
+
 // One axis pass of a complex transform over lines lm (in place).
 template <typename T, int DIR>
 void axis_c2c(const Fft1D<T>& p, cpx<T>* data, LineMap lm, T scale, cpx<T>* ws, hipStream_t st) {
@@ -34,15 +41,11 @@ void axis_c2c(const Fft1D<T>& p, cpx<T>* data, LineMap lm, T scale, cpx<T>* ws, 
         }
         return;
     }
-    if (p.single()) {
-        c2c_mapped<T, DIR>(p, data, data, lm, scale, st);
+    if (p.one_launch()) {
+        axis_one<T, DIR>(p, data, data, lm, scale, st);
         return;
     }
-    if (p.blue_single()) {
-        blue_mapped<T, DIR>(p, data, data, lm, scale, st);
-        return;
-    }
-    bool contig = lm.es == 1 && lm.s0 == p.n && lm.n0 >= lm.nlines;
+    bool contig = lm.es == 1 && lm.s0 == p.n && lm.div.mag == 0;
     if (contig) {
         c2c_contig<T, DIR>(p, data, data, lm.nlines, scale, ws, st);
         return;

@@ -205,6 +205,9 @@ __global__ void pair_out(IO io, const cpx<T>* __restrict__ y) {
     }
 }
 
+template <typename T>
+bool pair_one_launch(const Fft1D<T>& p) { return p.kind == K_GEN || p.blue_single(); }
+
 // Runs the lines lm through the n-point plan p; ws holds ceil(lines/2) * n
 // points plus p's workspace for them, unless p is one launch.
 template <typename T, int KIND, bool FWD>

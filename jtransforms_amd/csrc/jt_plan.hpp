@@ -49,6 +49,7 @@ struct jt_plan {
     bool pow2_all = false;
     // workspace (complex elements) each op touches; -1: op not defined
     int64_t op_ws[jt_api::NUM_OPS] = {-1, -1, -1, -1, -1, -1, -1, -1};
+    bool op_ws_used[jt_api::NUM_OPS] = {};
     // Calls on one plan are serialised: `mu` guards the host-side state (the
     // graph cache of ragged batches, flags) during a call, and the device work
     // of calls that touch the plan's buffers (workspace, staging, the ragged

@@ -461,6 +461,7 @@ struct R2R1D {
     std::unique_ptr<Fft1D<T>> full;  // n: lines in pairs
     DevBuf q, rtw;
     bool fused() const { return half && half->single(); }
+    bool one_launch() const { return n == 1 || fused() || (full && pair_one_launch(*full)); }
     int64_t ws_elems(int64_t lines) const {
         if (fused() || n == 1) return 0;
         // the bound that callers of the fixed-scratch entry point know: the

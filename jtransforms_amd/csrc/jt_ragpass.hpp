@@ -109,15 +109,15 @@ __global__ void __launch_bounds__(1024) ragged_pass(PArgs<T> a, const PItem* __r
     else if constexpr (KIND == PK_BLUE_S)
         run(IOListedBlue<T>{{a.data, a.off, a.tlist, scale}, c}, Fwd{});
     else if constexpr (KIND == PK_FOUR_A)
-        run(IOFourA<T, DIR>{x, w, hi, lo, n2, n, n1, n2, n1, 1, true}, D{});
+        run(IOFourA<T, DIR>{x, w, hi, lo, n2, n, n1, n2, n1, 1, true, LineDiv(n2, n2)}, D{});
     else if constexpr (KIND == PK_FOUR_B)
         run(IOStrided<T>{w, x, LineMap{n1, n1, 1, 0, n1}, n1, scale, true}, D{});
     else if constexpr (KIND == PK_BLUE_1)
-        run(IOBlueL<T, 1>{x, x, w, c, hi, lo, n2, n1, n2, scale, true}, Fwd{});
+        run(IOBlueL<T, 1>{x, x, w, c, hi, lo, n2, n1, n2, scale, true, LineDiv(n2, n2)}, Fwd{});
     else if constexpr (KIND == PK_BLUE_2)
-        run(IOBlueL<T, 2>{x, x, w, c, hi, lo, n1, n1, n2, scale, true}, Fwd{});
+        run(IOBlueL<T, 2>{x, x, w, c, hi, lo, n1, n1, n2, scale, true, LineDiv(n1, n1)}, Fwd{});
     else
-        run(IOBlueL<T, 3>{x, x, w, c, hi, lo, n2, n1, n2, scale, true}, Inv{});
+        run(IOBlueL<T, 3>{x, x, w, c, hi, lo, n2, n1, n2, scale, true, LineDiv(n2, n2)}, Inv{});
 }
 
 template <typename T>

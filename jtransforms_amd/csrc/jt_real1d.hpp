@@ -181,27 +181,44 @@ void real_inverse(const Real1D<T>& r, T* a, int64_t lines, bool scale, cpx<T>* w
                                      scale ? T(1.0 / (double)n) : T(1), ws, st);
 }
 
+// One launch from lines of n reals to their complex transforms, for a plan of
+// one launch.  A single line may be transformed onto itself (a workgroup has
+// read its lines before it writes).
+template <typename T, int DIR>
+void real_rows(const Fft1D<T>& p, const T* in, cpx<T>* out, int64_t lines, T scale, hipStream_t st) {
+    const IORealRows<T> io{in, out, p.n, lines, scale, false};
+    if (p.blue_single()) {
+        const Chirp<T> c{p.chirp.template as<cpx<T>>(), p.bspec.template as<cpx<T>>(), p.n, T(DIR)};
+        go_gen<T, -1>(*p.pm, IORealRowsBlue<T>{io, c}, false, st);
+    } else {
+        run_single<T, DIR, false>(p, io, st);
+    }
+}
+
 // realForwardFull / realInverseFull: complex transform of the real input
 // a[0..n) written as 2n values (dir -1 forward, +1 inverse with scale).
 template <typename T, int DIR>
-void real_full(const Real1D<T>& r, T* a, int64_t lines, bool scale, cpx<T>* ws, hipStream_t st) {
+void real_full(const Real1D<T>& r, T* a, bool scale, cpx<T>* ws, hipStream_t st) {
     const int64_t n = r.n;
-    if (lines <= 0) return;
-    // lines of the *input* are n reals apart in the reference's batched use
-    // (one line per call there), outputs 2n reals apart
-    cpx<T>* X = ws;
-    cpx<T>* ws2 = ws + lines * n;
+    const T s = (DIR > 0 && scale) ? T(1.0 / (double)n) : T(1);
+    cpx<T>* z = reinterpret_cast<cpx<T>*>(a);
+    if (r.full->one_launch()) {
+        real_rows<T, DIR>(*r.full, a, z, 1, s, st);
+        return;
+    }
     { JT_PROF(st, "real_to_complex");
-    hipLaunchKernelGGL((real_to_complex<T>), ew_grid(lines * n), dim3(256), 0, st, a, X, n, lines);
+    hipLaunchKernelGGL((real_to_complex<T>), ew_grid(n), dim3(256), 0, st, a, ws, n, (int64_t)1);
     }
     JT_HIP(hipGetLastError());
-    T s = (DIR > 0 && scale) ? T(1.0 / (double)n) : T(1);
-    c2c_contig<T, DIR>(*r.full, X, X, lines, s, ws2, st);
-    { JT_PROF(st, "copy_complex");
-    hipLaunchKernelGGL((copy_complex<T>), ew_grid(lines * n), dim3(256), 0, st, X,
-                       reinterpret_cast<cpx<T>*>(a), lines * n);
-    }
-    JT_HIP(hipGetLastError());
+    c2c_contig<T, DIR>(*r.full, ws, z, 1, s, ws + n, st);
 }
+
+// Instantiated in jt_full_f64.hip and jt_full_f32.hip.
+#define JT_FULL_INST1(X, T, D)                                                                            \
+    X template void real_rows<T, D>(const Fft1D<T>&, const T*, cpx<T>*, int64_t, T, hipStream_t);          \
+    X template void real_full<T, D>(const Real1D<T>&, T*, bool, cpx<T>*, hipStream_t);
+#define JT_FULL_INST(X, T) JT_FULL_INST1(X, T, -1) JT_FULL_INST1(X, T, 1)
+JT_FULL_INST(extern, float)
+JT_FULL_INST(extern, double)
 
 }  // namespace jt

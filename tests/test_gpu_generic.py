@@ -161,3 +161,30 @@ def test_odd_packed_batch(orc, n, prec):
         for b in range(lines):
             s = slice(b * n, (b + 1) * n)
             assert rel(c[s], orc.real_inverse(n, x[s].astype(np.float64), scale)) <= 2 * tol(n, prec), (b, scale)
+
+
+# single-launch, Bluestein and several-launch plans on each axis
+FULL = [(2,), (16,), (37,), (360,), (4096,), (2047,), (4103,), (10158,), (2, 2), (9, 37), (37, 16), (64, 225),
+        (4103, 3), (3, 4103), (5, 6, 7), (16, 37, 9), (3, 4, 10158)]
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("dims", FULL)
+def test_real_full(orc, dims, prec):
+    """realForwardFull / realInverseFull(scale) where the row pass reads the
+    reals, and where it cannot."""
+    tot = int(np.prod(dims))
+    x = orc.jrandom_doubles(tot, tot).astype(DT[prec])
+    src = np.concatenate([x, np.zeros_like(x)])
+    cls = [{"f64": jt.DoubleFFT_1D, "f32": jt.FloatFFT_1D}, FFT2, {"f64": jt.DoubleFFT_3D, "f32": jt.FloatFFT_3D}]
+    p = cls[len(dims) - 1][prec](*dims)
+    z = (x.astype(np.float64) + 0j).reshape(dims)
+    for fwd in (True, False):
+        a = src.copy()
+        if fwd:
+            p.realForwardFull(a)
+        else:
+            p.realInverseFull(a, True)
+        want = np.fft.fftn(z) if fwd else np.fft.ifftn(z)
+        e = rel(a, np.ascontiguousarray(want).view(np.float64))
+        assert e <= tol(tot, prec), (fwd, e)
