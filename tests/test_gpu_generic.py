@@ -188,3 +188,43 @@ def test_real_full(orc, dims, prec):
         want = np.fft.fftn(z) if fwd else np.fft.ifftn(z)
         e = rel(a, np.ascontiguousarray(want).view(np.float64))
         assert e <= tol(tot, prec), (fwd, e)
+
+
+def test_device_calls_after_the_first(orc):
+    """Later calls of a plan on flat device tensors take the short path: the
+    same results, streams, offsets and refusals as the first."""
+    import torch
+    n = 600
+    x = orc.jrandom_doubles(n, 2 * n + 3)
+    p = jt.DoubleFFT_1D(n)
+    want = orc.complex_forward(n, x[:2 * n])
+    s = torch.cuda.Stream()
+    for rep in range(3):
+        t = torch.from_numpy(x.copy()).cuda()
+        torch.cuda.synchronize()
+        if rep == 2:
+            with torch.cuda.stream(s):
+                p.complexForward(t)
+            s.synchronize()
+        else:
+            p.complexForward(t)
+        y = t.cpu().numpy()
+        assert rel(y[:2 * n], want) <= tol(n, "f64") and np.array_equal(y[2 * n:], x[2 * n:])
+    t = torch.from_numpy(x.copy()).cuda()
+    p.complexForward(t, 3)  # misaligned pairs
+    assert rel(t.cpu().numpy()[3:], orc.complex_forward(n, x[3:])) <= tol(n, "f64")
+    good = torch.zeros(2 * n, dtype=torch.float64, device="cuda")
+    with pytest.raises(TypeError):
+        p.complexForward(good.float())
+    with pytest.raises(TypeError):
+        p.complexForward(good.cpu())
+    with pytest.raises(TypeError):
+        p.complexForward(torch.zeros(4 * n, dtype=torch.float64, device="cuda")[::2])
+    with pytest.raises(TypeError):
+        p.complexForward(good.reshape(2, n))
+    with pytest.raises(IndexError):
+        p.complexForward(good[:-1])
+    with pytest.raises(IndexError):
+        p.complexForward(good, 1)
+    with pytest.raises(ValueError):
+        p.complexForward(good, -1)
