@@ -549,6 +549,28 @@ void go_tpl(IO io, const cpx<T>* tw, hipStream_t st) {
             return;
         }
     }
+    if constexpr (COL && !REAL && !HOOKS && N >= 256 && S::W >= 8) {
+        // Columns too few to give each of the 256 CUs a workgroup: half as
+        // many per workgroup below 192 workgroups, a quarter up to 64 (whole
+        // calls in both directions, us, full : half : quarter width).
+        //   64 and fewer: real 1024^2 FP32 39.5 : 33.3 : 30.0, real 512^2
+        //     FP64 29.5 : 25.8 : 23.8, 512^2 FP32 24.2 : 21.4 : 20.6,
+        //     256^2 FP64 20.4 : 19.4 : 18.8
+        //   128: 1024^2 FP64 49.9 : 45.6 : 49.1, real 2048^2 FP32 69.9 :
+        //     62.6 : 65.9
+        //   256: real 4096 x 2048 FP32 88.6 : 94.3, 2048 x 1024 FP64 64.7 : 67.8
+        const int64_t groups = (io.nlines + S::W - 1) / S::W;
+        if (groups < 192) {
+            constexpr int W2 = S::W / 2, W4 = S::W / 4;
+            if (groups <= 64)
+                launch_tpl<T, DIR, N, TL, W4, COL, (2 * LdsGeom<N, W4>::size * (int)sizeof(T) > 65536), IO, Rs...>(io, tw,
+                                                                                                               st);
+            else
+                launch_tpl<T, DIR, N, TL, W2, COL, (2 * LdsGeom<N, W2>::size * (int)sizeof(T) > 65536), IO, Rs...>(io, tw,
+                                                                                                               st);
+            return;
+        }
+    }
     if constexpr (!COL && REAL && TL <= 16) {
         // short rows of reals (DCT/DST/DHT x axis): one wave per workgroup
         // (512^3 FP64 DCT row pass, 16 -> 8 -> 4 -> 2 lines per workgroup:

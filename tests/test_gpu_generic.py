@@ -228,3 +228,24 @@ def test_device_calls_after_the_first(orc):
         p.complexForward(good, 1)
     with pytest.raises(ValueError):
         p.complexForward(good, -1)
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("rows,cols", [(256, 3), (256, 1030), (512, 520), (1024, 515), (1024, 1030), (2048, 129),
+                                       (4096, 65), (2048, 1024)])
+def test_narrow_column_groups(orc, rows, cols, prec):
+    """Compile-time columns in groups of full, half and quarter width, with a
+    partly filled last group; the packed real form where cols allows."""
+    x = orc.jrandom_doubles(rows + cols, 2 * rows * cols).astype(DT[prec])
+    p = FFT2[prec](rows, cols)
+    a = x.copy()
+    p.complexForward(a)
+    assert rel(a, orc.fftnd_complex([rows, cols], x.astype(np.float64), -1)) <= tol(rows * cols, prec)
+    p.complexInverse(a, True)
+    assert rel(a, x) <= 2 * tol(rows * cols, prec)
+    if cols & (cols - 1) == 0:
+        r = x[:rows * cols].copy()
+        p.realForward(r)
+        assert rel(r, orc.fft2d_real_forward(rows, cols, x[:rows * cols].astype(np.float64))) <= tol(rows * cols, prec)
+        p.realInverse(r, True)
+        assert rel(r, x[:rows * cols]) <= 2 * tol(rows * cols, prec)
