@@ -233,7 +233,10 @@ __global__ void __launch_bounds__(TL* W) stockham_kernel(IO io, const cpx<T>* __
     LdsBuf<T, N, W, SPLIT> lds{lds_re, lds_im};
 
     const int tid = threadIdx.x;
-    const int w = COLMODE ? tid % W : tid / TL;
+    // (a row that fills whole waves: its line, and the line's offset, are
+    // scalar.  Per lane, the offset's multiplications took the 16384 x 4096
+    // FP32 batch from 184 to 188 us a direction)
+    const int w = COLMODE ? tid % W : TL % 64 == 0 ? __builtin_amdgcn_readfirstlane(tid / TL) : tid / TL;
     const int t = COLMODE ? tid / W : tid % TL;
     const int64_t ngroups = (io.nlines + W - 1) / W;
     const int64_t g = io.xcd ? xcd_group(blockIdx.x, ngroups) : (int64_t)blockIdx.x;
