@@ -1,6 +1,6 @@
 // Real transforms of lengths without a fused half-length plan (odd n, even n
-// whose half has a large prime factor): two real lines travel as the real and
-// imaginary part of one n-point complex transform,
+// whose half has a large prime factor).  In a DCT, DST or DHT two real lines
+// travel as the real and imaginary part of one n-point complex transform,
 //   Z = DFT(v_a + i v_b),  V_a = (Z_k + conj Z_{n-k})/2,
 //                          V_b = (Z_k - conj Z_{n-k})/2i,
 // in one launch while n (or its Bluestein convolution) fits a workgroup's
@@ -9,6 +9,10 @@
 // It replaces a mirrored 2n-point complex transform of every line: a quarter
 // of the points (DST 999 x 1000 FP64, both directions: 203 -> 97 us; DST
 // 381 x 1099 FP32 333 -> 64 with one-launch Bluestein).
+// Two such lines share their rounding errors and their NaNs, which is right
+// where several lines exist only as an axis of a 2D or 3D transform, whose
+// other axes mix them all.  The lines of a batch of packed real transforms are
+// signals of their own: they travel one by one, with zero imaginary parts.
 #pragma once
 #include "jt_fft1d.hpp"
 
@@ -23,8 +27,9 @@ template <typename T, int KIND, bool FWD, bool CONV, typename I = int>
 struct IOPair {
     static constexpr bool pre_lds = true, post_lds = true, store_loads = false, conv = CONV;
     static constexpr bool makhoul = KIND == R2R_DCT || KIND == R2R_DST;
+    static constexpr bool paired = KIND != R2R_PACKED;
     static const char* tag() {
-        return KIND == R2R_DHT ? "dht,pair" : KIND == R2R_PACKED ? (FWD ? "r2c,pair" : "c2r,pair")
+        return KIND == R2R_DHT ? "dht,pair" : KIND == R2R_PACKED ? (FWD ? "r2c,odd" : "c2r,odd")
                : KIND == R2R_DCT ? (FWD ? "dct2,pair" : "dct3,pair") : (FWD ? "dst2,pair" : "dst3,pair");
     }
     std::string desc() const { return ",n=" + std::to_string(n) + ",es=" + std::to_string(m.es); }
@@ -32,7 +37,7 @@ struct IOPair {
     const cpx<T>* q;  // DCT, DST: exp(-i pi k / 2n), k in [0, n]
     Chirp<T> c;       // CONV
     LineMap m;
-    int64_t nlines;  // pairs
+    int64_t nlines;  // transforms: pairs, or single lines
     I n;
     int len;  // points of the LDS line: n, or the convolution's m
     T f0, g;
@@ -42,17 +47,24 @@ struct IOPair {
         bool two;  // the last pair of an odd number of lines has one
     };
     __device__ __forceinline__ At base(int64_t p) const {
+        if constexpr (!paired) {
+            const int64_t o = m.base(p);
+            return At{o, o, false};
+        }
         const int64_t a = m.base(2 * p);
         const bool two = 2 * p + 1 < m.nlines;
         return At{a, two ? m.base(2 * p + 1) : a, two};
     }
     __device__ __forceinline__ cpx<T> rd(At at, I i) const {
+        if constexpr (!paired) return cpx<T>{data[at.a + i * m.es], T(0)};
         const cpx<T> v{data[at.a + i * m.es], data[at.b + i * m.es]};
         return cpx<T>{v.x, at.two ? v.y : T(0)};
     }
     __device__ __forceinline__ void wr(At at, I i, T a, T b) const {
         data[at.a + i * m.es] = a;
-        if (at.two) data[at.b + i * m.es] = b;
+        if constexpr (paired) {
+            if (at.two) data[at.b + i * m.es] = b;
+        }
     }
     // the line's element that is v_j
     __device__ __forceinline__ I vidx(I j) const {
@@ -179,7 +191,7 @@ struct IOPair {
 };
 
 // The same steps around a transform of several launches, through a workspace
-// of one n-point line per pair.
+// of one n-point line per transform.
 template <typename T, class IO>
 __global__ void pair_in(IO io, cpx<T>* __restrict__ y) {
     const int64_t n = io.n, tot = io.nlines * n;
@@ -208,31 +220,32 @@ __global__ void pair_out(IO io, const cpx<T>* __restrict__ y) {
 template <typename T>
 bool pair_one_launch(const Fft1D<T>& p) { return p.kind == K_GEN || p.blue_single(); }
 
-// Runs the lines lm through the n-point plan p; ws holds ceil(lines/2) * n
-// points plus p's workspace for them, unless p is one launch.
+// Runs the lines lm through the n-point plan p; ws holds n points per
+// transform (a pair of lines, or a line if packed) plus p's workspace for
+// them, unless p is one launch.
 template <typename T, int KIND, bool FWD>
 void pair_lines(const Fft1D<T>& p, T* data, const cpx<T>* q, LineMap lm, T f0, T g, cpx<T>* ws, hipStream_t st) {
-    const int64_t pairs = (lm.nlines + 1) / 2;
+    const int64_t count = KIND == R2R_PACKED ? lm.nlines : (lm.nlines + 1) / 2;
     constexpr int D = FWD ? -1 : 1;
     const bool col = lm.es != 1;
     if (p.kind == K_GEN) {
-        go_gen<T, D>(p, IOPair<T, KIND, FWD, false>{data, q, {}, lm, pairs, (int)p.n, (int)p.n, f0, g, col}, col, st);
+        go_gen<T, D>(p, IOPair<T, KIND, FWD, false>{data, q, {}, lm, count, (int)p.n, (int)p.n, f0, g, col}, col, st);
         return;
     }
     if (p.blue_single()) {
         const Chirp<T> c{p.chirp.template as<cpx<T>>(), p.bspec.template as<cpx<T>>(), p.n, T(D)};
-        go_gen<T, -1>(*p.pm, IOPair<T, KIND, FWD, true>{data, q, c, lm, pairs, (int)p.n, (int)p.m, f0, g, col}, col, st);
+        go_gen<T, -1>(*p.pm, IOPair<T, KIND, FWD, true>{data, q, c, lm, count, (int)p.n, (int)p.m, f0, g, col}, col, st);
         return;
     }
     using IO = IOPair<T, KIND, FWD, false, int64_t>;
-    const IO io{data, q, {}, lm, pairs, p.n, 0, f0, g, false};
+    const IO io{data, q, {}, lm, count, p.n, 0, f0, g, false};
     { JT_PROF(st, "pair_in");
-    hipLaunchKernelGGL((pair_in<T, IO>), ew_grid(pairs * p.n), dim3(256), 0, st, io, ws);
+    hipLaunchKernelGGL((pair_in<T, IO>), ew_grid(count * p.n), dim3(256), 0, st, io, ws);
     }
     JT_HIP(hipGetLastError());
-    c2c_contig<T, D>(p, ws, ws, pairs, T(1), ws + pairs * p.n, st);
+    c2c_contig<T, D>(p, ws, ws, count, T(1), ws + count * p.n, st);
     { JT_PROF(st, "pair_out");
-    hipLaunchKernelGGL((pair_out<T, IO, FWD>), ew_grid(pairs * (FWD ? p.n / 2 + 1 : p.n)), dim3(256), 0, st, io, ws);
+    hipLaunchKernelGGL((pair_out<T, IO, FWD>), ew_grid(count * (FWD ? p.n / 2 + 1 : p.n)), dim3(256), 0, st, io, ws);
     }
     JT_HIP(hipGetLastError());
 }

@@ -142,7 +142,7 @@ void real_forward(const Real1D<T>& r, T* a, int64_t lines, cpx<T>* ws, hipStream
         }
         return;
     }
-    // odd n
+    // odd n (a line per transform)
     pair_lines<T, R2R_PACKED, true>(*r.full, a, nullptr, LineMap{lines, lines, n, 0, 1}, T(1), T(1), ws, st);
 }
 

@@ -163,6 +163,35 @@ def test_odd_packed_batch(orc, n, prec):
             assert rel(c[s], orc.real_inverse(n, x[s].astype(np.float64), scale)) <= 2 * tol(n, prec), (b, scale)
 
 
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("n", [3, 9, 37, 225, 1021, 4095, 4103, 33075, 74, 1000, 2042, 4096, 20000])
+def test_packed_batch_lines_are_independent(orc, n, prec):
+    """The lines of a batch are signals of their own: a line 10^16 times as
+    loud as another, or one with a NaN or an infinity, leaves the others what
+    they are alone, to the last bit."""
+    lines, amp = 5, [1.0, 1e-8, 1e8, 1e-8, 1.0]
+    x = orc.jrandom_doubles(n + 1, n * lines).astype(DT[prec]).reshape(lines, n)
+    x *= np.array(amp, DT[prec])[:, None]
+    p = jt.FFTBatch1D(n, lines, precision=prec)
+    ops = {"forward": (lambda a: p.realForward(a), orc.real_forward, ()),
+           "inverse": (lambda a: p.realInverse(a, True), orc.real_inverse, (True,))}
+    for op, (call, ref, more) in ops.items():
+        a = x.reshape(-1).copy()
+        call(a)
+        a = a.reshape(lines, n)
+        for b in range(lines):
+            e = rel(a[b], ref(n, x[b].astype(np.float64), *more))
+            assert e <= 2 * tol(n, prec), (op, b, e)
+        y = x.copy()
+        y[1, n // 2], y[2, 0] = np.nan, np.inf
+        y = y.reshape(-1)
+        call(y)
+        y = y.reshape(lines, n)
+        for b in (0, 3, 4):
+            assert np.array_equal(y[b], a[b]), (op, b)
+        assert not np.isfinite(y[1]).all() and not np.isfinite(y[2]).all(), op
+
+
 # single-launch, Bluestein and several-launch plans on each axis
 FULL = [(2,), (16,), (37,), (360,), (4096,), (2047,), (4103,), (10158,), (2, 2), (9, 37), (37, 16), (64, 225),
         (4103, 3), (3, 4103), (5, 6, 7), (16, 37, 9), (3, 4, 10158)]
