@@ -62,8 +62,8 @@ enum {
     /* ragged batches: capture the launch sequence in a hipGraph on the first
      * call for a given (data, stream, op) and replay it afterwards */
     JT_FLAG_GRAPH = 2,
-    /* ragged batches: choose the schedule (LDS split, tile shape, work-item
-     * size, radix order) by timing candidate plans at creation; the choice is
+    /* ragged batches: choose the schedule (form, LDS split, tile shape,
+     * work-item size, radix order) by timing candidate plans at creation; the choice is
      * remembered for the same length list within the process */
     JT_FLAG_AUTOTUNE = 4
 };

@@ -317,9 +317,10 @@ std::unique_ptr<RaggedPlan<T>> make_ragged_tuned(const int64_t* lengths, int64_t
                                                  std::string* desc) {
     std::unique_ptr<RaggedPlan<T>> P;
     if (!tune) {
-        // JT_RAGGED_SCHEDULE="wgs=2,nt=512,tplx=0,chunk=8,order=0,lag=16" (any
-        // subset; the format of jt_plan_describe) fixes the schedule of
-        // untuned plans, for tests and measurements of one schedule
+        // JT_RAGGED_SCHEDULE="wgs=2,nt=512,tplx=0,chunk=8,order=0,lag=16,
+        // form=persistent" (any subset; the format of jt_plan_describe) fixes
+        // the schedule of untuned plans, to reuse a tuned one or to test and
+        // measure one schedule; form is persistent unless it says launches
         RTune t;
         if (const char* e = std::getenv("JT_RAGGED_SCHEDULE")) {
             std::string sch(e);
@@ -331,8 +332,13 @@ std::unique_ptr<RaggedPlan<T>> make_ragged_tuned(const int64_t* lengths, int64_t
                 const size_t eq = kv.find('=');
                 if (eq != std::string::npos) {
                     const std::string k = kv.substr(0, eq);
-                    const int v = std::atoi(kv.c_str() + eq + 1);
-                    if (k == "wgs") t.wgs = v;
+                    const std::string val = kv.substr(eq + 1);
+                    const int v = std::atoi(val.c_str());
+                    if (k == "form") {
+                        if (val != "persistent" && val != "launches")
+                            throw JtError(ST_BAD_ARG, "JT_RAGGED_SCHEDULE: form is persistent or launches, not " + val);
+                        t.form = val == "launches" ? 1 : 0;
+                    } else if (k == "wgs") t.wgs = v;
                     else if (k == "nt") t.nt = v;
                     else if (k == "tplx") t.tplx = v;
                     else if (k == "chunk") t.chunk = v;

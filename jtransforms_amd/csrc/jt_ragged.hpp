@@ -113,9 +113,11 @@ struct RArgs {
 struct RTune {
     int wgs = 2, nt = 0, tplx = 0, chunk = 4, order = 0, lag = 0;  // nt 0: smallest that fits
     int form = 0;
+    // what jt_plan_describe prints and JT_RAGGED_SCHEDULE takes
     std::string str() const {
         return "wgs=" + std::to_string(wgs) + ",nt=" + std::to_string(nt) + ",tplx=" + std::to_string(tplx) +
-               ",chunk=" + std::to_string(chunk) + ",order=" + std::to_string(order) + ",lag=" + std::to_string(lag) + (form ? ",form=launches" : "");
+               ",chunk=" + std::to_string(chunk) + ",order=" + std::to_string(order) + ",lag=" + std::to_string(lag) +
+               ",form=" + (form ? "launches" : "persistent");
     }
     bool operator==(const RTune& o) const {
         return wgs == o.wgs && nt == o.nt && tplx == o.tplx && chunk == o.chunk && order == o.order && lag == o.lag &&

@@ -88,3 +88,14 @@ def test_ragged_schedule_override_range_checked(monkeypatch, sched):
     monkeypatch.setenv("JT_RAGGED_SCHEDULE", sched)
     with pytest.raises(ValueError, match="ragged schedule out of range"):
         jt.RaggedBatch1D(np.array([16, 32], dtype=np.int64))
+
+
+def test_ragged_schedule_override_form(monkeypatch):
+    """The form is one of the two that descriptions name."""
+    import numpy as np
+    monkeypatch.setenv("JT_RAGGED_SCHEDULE", "wgs=2,form=bogus")
+    with pytest.raises(ValueError, match="form is persistent or launches, not bogus"):
+        jt.RaggedBatch1D(np.array([16, 32], dtype=np.int64))
+    monkeypatch.setenv("JT_RAGGED_SCHEDULE", "form=launches,chunk=0")
+    with pytest.raises(ValueError, match="ragged schedule out of range"):
+        jt.RaggedBatch1D(np.array([16, 32], dtype=np.int64))

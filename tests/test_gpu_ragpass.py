@@ -51,3 +51,35 @@ def test_passes(orc, prec):
     for i, n in enumerate(lens):
         assert rel(z[seg[i]], x[seg[i]]) <= 2 * tol(n, prec), (i, n)
         assert rel(w[seg[i]], float(n) * x[seg[i]].astype(np.float64)) <= 2 * tol(n, prec), (i, n)
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("form", ["persistent", "launches"])
+@pytest.mark.parametrize("big", [False, True])
+def test_described_schedule_is_accepted(orc, form, big, prec, monkeypatch):
+    """JT_RAGGED_SCHEDULE takes what describe() prints, of either form, and
+    gives the same schedule for batches on both sides of the default's line;
+    tuned plans describe theirs the same way."""
+    import torch
+    lens = np.array([12800, 10007, 17, 17, 360, 4096] + ([65536, 65521] if big else []), dtype=np.int64)
+    monkeypatch.setenv("JT_RAGGED_SCHEDULE", "form=" + form)
+    first = jt.RaggedBatch1D(lens, precision=prec).describe()
+    assert "form=" + form in first, first
+    sched = first.split("schedule ")[1].split()[0]
+    monkeypatch.setenv("JT_RAGGED_SCHEDULE", sched)
+    p = jt.RaggedBatch1D(lens, precision=prec)
+    assert p.describe() == first
+    x = orc.jrandom_doubles(20110630, int(2 * lens.sum())).astype(DT[prec])
+    t = torch.from_numpy(x.copy()).cuda()
+    p.complexForward(t)
+    y = t.cpu().numpy()
+    p.sync_status()
+    for i, n in enumerate(lens):
+        s = slice(int(p.offsets[i]), int(p.offsets[i + 1]))
+        assert rel(y[s], orc.complex_forward(int(n), x[s].astype(np.float64))) <= tol(n, prec), (i, n)
+    if form == "launches" and not big:
+        monkeypatch.delenv("JT_RAGGED_SCHEDULE")
+        tuned = jt.RaggedBatch1D(lens, precision=prec, autotune=True).describe()
+        sched = tuned.split("schedule ")[1].split()[0]
+        monkeypatch.setenv("JT_RAGGED_SCHEDULE", sched)
+        assert jt.RaggedBatch1D(lens, precision=prec).describe().split("schedule ")[1].split()[0] == sched
