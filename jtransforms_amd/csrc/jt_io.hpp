@@ -4,35 +4,11 @@
 #include <string>
 
 #include "jt_dft.hpp"
+#include "jt_linemap.hpp"
 
 namespace jt {
 
 __device__ __forceinline__ int lpos(int k) { return k + (k >> 5); }
-
-// l / n0 for 0 <= l < nlines as a multiply by mag = floor(2^64 / n0) + 1
-// (exact while l * n0 < 2^64); mag 0 where the quotient is always 0.  Straight
-// code: a 64-bit division takes over a hundred instructions, and a branch
-// around it puts the kernel arguments behind it a second, late load.
-struct LineDiv {
-    int64_t n0;
-    uint64_t mag;
-    __host__ __device__ LineDiv(int64_t nlines, int64_t d) : n0(d), mag(nlines <= d ? 0 : ~uint64_t(0) / d + 1) {}
-    __device__ __forceinline__ int64_t operator()(int64_t l) const { return (int64_t)__umul64hi((uint64_t)l, mag); }
-};
-
-// Lines l in [0, nlines) start at (l % n0)*s0 + (l / n0)*s1 (complex units);
-// element k of a line sits es further per step.  (n0 = 1 is the same as
-// n0 = nlines with s0 = s1.)
-struct LineMap {
-    int64_t nlines, s0, s1, es;
-    LineDiv div;
-    __host__ __device__ LineMap(int64_t nl, int64_t n0, int64_t s0_, int64_t s1_, int64_t es_)
-        : nlines(nl), s0(n0 == 1 ? s1_ : s0_), s1(s1_), es(es_), div(nl, n0 == 1 ? nl : n0) {}
-    __device__ __forceinline__ int64_t base(int64_t l) const {
-        const int64_t q = div(l);
-        return (l - q * div.n0) * s0 + q * s1;
-    }
-};
 
 // Non-temporal (streaming) complex loads and stores: they skip the caches'
 // allocation, which lets a pass that reads or writes each element once run

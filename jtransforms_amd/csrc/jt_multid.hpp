@@ -28,8 +28,10 @@ __global__ void scatter_lines(const cpx<T>* __restrict__ y, cpx<T>* __restrict__
 // One axis pass over lines lm from `in` to `out`, for a plan of one launch.
 template <typename T, int DIR>
 void axis_one(const Fft1D<T>& p, const cpx<T>* in, cpx<T>* out, LineMap lm, T scale, hipStream_t st) {
-    if (p.single()) c2c_mapped<T, DIR>(p, in, out, lm, scale, st);
-    else blue_mapped<T, DIR>(p, in, out, lm, scale, st);
+    exact_maps(lm, [&](int64_t off, const LineMap& m) {
+        if (p.single()) c2c_mapped<T, DIR>(p, in + off, out + off, m, scale, st);
+        else blue_mapped<T, DIR>(p, in + off, out + off, m, scale, st);
+    });
 }
 
 // One axis pass of a complex transform over lines lm (in place).
@@ -48,6 +50,10 @@ void axis_c2c(const Fft1D<T>& p, cpx<T>* data, LineMap lm, T scale, cpx<T>* ws, 
     bool contig = lm.es == 1 && lm.s0 == p.n && lm.div.mag == 0;
     if (contig) {
         c2c_contig<T, DIR>(p, data, data, lm.nlines, scale, ws, st);
+        return;
+    }
+    if (!lm.div.exact(lm.nlines)) {
+        exact_maps(lm, [&](int64_t off, const LineMap& m) { axis_c2c<T, DIR>(p, data + off, m, scale, ws, st); });
         return;
     }
     cpx<T>* g = ws;

@@ -537,6 +537,10 @@ template <typename T>
 void r2r_axis(int family, const R2R1D<T>& r, T* data, LineMap lm, bool fwd, bool scale, cpx<T>* ws,
               hipStream_t st) {
     if (r.n == 1 || lm.nlines <= 0) return;
+    if (!lm.div.exact(lm.nlines)) {
+        exact_maps(lm, [&](int64_t off, const LineMap& m) { r2r_axis<T>(family, r, data + off, m, fwd, scale, ws, st); });
+        return;
+    }
     if (family == 1) {
         if (fwd) r2r_axis_k<T, R2R_DCT, true>(r, data, lm, scale, ws, st);
         else r2r_axis_k<T, R2R_DCT, false>(r, data, lm, scale, ws, st);
