@@ -158,13 +158,12 @@ int execute_locked(jt_plan* p, int op, char* ptr, int scale, hipStream_t st) {
         d = staging_area(p, op);
         JT_HIP(hipMemcpyAsync(d, ptr, bytes, hipMemcpyDeviceToDevice, st));
     }
+    char* ws = p->op_ws_used[op] ? ws_base(p) : nullptr;
     int rc;
     if (p->precision == JT_F64)
-        rc = exec_t<double>(p, op, reinterpret_cast<double*>(d), scale != 0,
-                            reinterpret_cast<cpx<double>*>(ws_base(p)), st);
+        rc = exec_t<double>(p, op, reinterpret_cast<double*>(d), scale != 0, reinterpret_cast<cpx<double>*>(ws), st);
     else
-        rc = exec_t<float>(p, op, reinterpret_cast<float*>(d), scale != 0,
-                           reinterpret_cast<cpx<float>*>(ws_base(p)), st);
+        rc = exec_t<float>(p, op, reinterpret_cast<float*>(d), scale != 0, reinterpret_cast<cpx<float>*>(ws), st);
     if (rc == JT_OK && staged) JT_HIP(hipMemcpyAsync(ptr, d, bytes, hipMemcpyDeviceToDevice, st));
     if (chained) {
         JT_HIP(hipEventRecord(p->chain, st));
@@ -354,6 +353,7 @@ int jt_execute_noalloc(jt_plan* p, int op, void* data, int64_t offset, int scale
             d = ws + (size_t)p->op_ws[op] * cs;
             JT_HIP(hipMemcpyAsync(d, ptr, bytes, hipMemcpyDeviceToDevice, st));
         }
+        if (!p->op_ws_used[op]) ws = nullptr;
         int rc;
         if (p->precision == JT_F64)
             rc = exec_t<double>(p, op, reinterpret_cast<double*>(d), scale != 0, reinterpret_cast<cpx<double>*>(ws),

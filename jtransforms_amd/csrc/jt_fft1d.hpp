@@ -857,6 +857,16 @@ template <typename T, int DIR>
 void c2c_contig(const Fft1D<T>& p, const cpx<T>* in, cpx<T>* out, int64_t lines, T scale,
                 cpx<T>* ws, hipStream_t st);
 
+// The workspace of a path that uses one.  A call that was taken to use none
+// (so that it is not ordered after other streams' calls of its plan) is handed
+// null: a path that needs the workspace all the same fails here, on the host,
+// instead of racing for it.
+template <typename T>
+cpx<T>* need_ws(cpx<T>* ws) {
+    if (!ws) throw JtError(ST_UNSUPPORTED, "internal: a path uses the workspace that its op does not declare");
+    return ws;
+}
+
 // arrays at least this large are streamed (non-temporal) by first/last passes
 constexpr int64_t NT_MIN_BYTES = int64_t(64) << 20;
 
@@ -900,6 +910,7 @@ void c2c_contig(const Fft1D<T>& p, const cpx<T>* in, cpx<T>* out, int64_t lines,
         return;
     }
     if (p.kind == K_FOUR) {
+        need_ws(ws);
         if (!p.p1->single()) throw JtError(ST_UNSUPPORTED, "four-step column plan must be single-kernel");
         const bool two = p.p2->single();
         IOFourA<T, DIR> a{in, ws, p.hi.template as<cpx<T>>(), p.lo.template as<cpx<T>>(), lines * p.n2,
@@ -928,6 +939,7 @@ void c2c_contig(const Fft1D<T>& p, const cpx<T>* in, cpx<T>* out, int64_t lines,
         blue_mapped<T, DIR>(p, in, out, LineMap{lines, lines, p.n, 0, 1}, scale, st);
         return;
     }
+    need_ws(ws);
     if (p.pb) {
         const Fft1D<T>& f = *p.pm;
         const Chirp<T> c{p.chirp.template as<cpx<T>>(), p.bspec.template as<cpx<T>>(), p.n, T(DIR)};

@@ -48,7 +48,8 @@ int64_t op_ws_need(jt_plan* p, int op) {
 }
 
 // Whether op touches its workspace at all (op_ws_need is a bound that also
-// holds for the fixed-scratch entry point).
+// holds for the fixed-scratch entry point).  The paths below hold this to its
+// word: without it they get no workspace (need_ws).
 template <typename T>
 bool op_uses_ws(jt_plan* p, int op) {
     Impl<T>& I = impl<T>(p);
@@ -205,6 +206,7 @@ void run_real_inverse_nd(jt_plan* p, T* a, bool scale, cpx<T>* ws, hipStream_t s
 // input (first prod(dims) elements), written as interleaved complex.
 template <typename T, int DIR>
 void run_real_full_nd(jt_plan* p, T* a, bool scale, cpx<T>* ws, hipStream_t st) {
+    need_ws(ws);
     const int64_t tot = total(p);
     Impl<T>& I = impl<T>(p);
     const int nd = p->ndim;

@@ -56,7 +56,7 @@ void axis_c2c(const Fft1D<T>& p, cpx<T>* data, LineMap lm, T scale, cpx<T>* ws, 
         exact_maps(lm, [&](int64_t off, const LineMap& m) { axis_c2c<T, DIR>(p, data + off, m, scale, ws, st); });
         return;
     }
-    cpx<T>* g = ws;
+    cpx<T>* g = need_ws(ws);
     cpx<T>* ws2 = ws + lm.nlines * p.n;
     { JT_PROF(st, "gather_lines");
     hipLaunchKernelGGL((gather_lines<T>), ew_grid(lm.nlines * p.n), dim3(256), 0, st, data, g, lm, p.n);

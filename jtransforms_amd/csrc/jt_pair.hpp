@@ -237,6 +237,7 @@ void pair_lines(const Fft1D<T>& p, T* data, const cpx<T>* q, LineMap lm, T f0, T
         go_gen<T, -1>(*p.pm, IOPair<T, KIND, FWD, true>{data, q, c, lm, count, (int)p.n, (int)p.m, f0, g, col}, col, st);
         return;
     }
+    need_ws(ws);
     using IO = IOPair<T, KIND, FWD, false, int64_t>;
     const IO io{data, q, {}, lm, count, p.n, 0, f0, g, false};
     { JT_PROF(st, "pair_in");

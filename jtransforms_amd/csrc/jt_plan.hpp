@@ -114,7 +114,7 @@ void build(jt_plan* p);
 template <typename T>
 void apply_flags(Impl<T>& I, uint32_t flags);
 // runs `op` on pair-aligned device data `a`; `ws` is the op's workspace
-// (op_ws[op] complex elements)
+// (op_ws[op] complex elements), null if it uses none (op_ws_used)
 template <typename T>
 int exec_t(jt_plan* p, int op, T* a, bool scale, cpx<T>* ws, hipStream_t st);
 template <typename T>

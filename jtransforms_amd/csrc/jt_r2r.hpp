@@ -518,6 +518,7 @@ void r2r_axis_k(const R2R1D<T>& r, T* data, LineMap lm, bool scale, cpx<T>* ws, 
         pair_lines<T, KIND, FWD>(*r.full, data, q, lm, f0, g, ws, st);
         return;
     }
+    need_ws(ws);
     const cpx<T>* rtw = r.rtw.template as<cpx<T>>();
     const int64_t N = n / 2;
     constexpr int D = FWD || KIND == R2R_DHT ? -1 : 1;

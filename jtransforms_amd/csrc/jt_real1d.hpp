@@ -206,6 +206,7 @@ void real_full(const Real1D<T>& r, T* a, bool scale, cpx<T>* ws, hipStream_t st)
         real_rows<T, DIR>(*r.full, a, z, 1, s, st);
         return;
     }
+    need_ws(ws);
     { JT_PROF(st, "real_to_complex");
     hipLaunchKernelGGL((real_to_complex<T>), ew_grid(n), dim3(256), 0, st, a, ws, n, (int64_t)1);
     }

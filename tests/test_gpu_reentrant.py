@@ -90,6 +90,53 @@ def test_two_streams_share_one_plan(orc, n, offa):
         assert rel(b.cpu().numpy(), xs[i]) <= 2 * tol(n), i
 
 
+# forms that use the plan's workspace and forms that do not, neighbours of the
+# line between them: Bluestein in one launch and in three, odd and half-length
+# real transforms of one launch and of several, the expanded real transforms
+SHARED = [("c2c", (1021,)), ("c2c", (4103,)), ("c2c", (37, 1021)), ("c2c", (6, 10007)), ("real", (999,)),
+          ("real", (1021,)), ("real", (33075,)), ("real", (2042,)), ("real", (20000,)), ("real", (64, 128)),
+          ("full", (360,)), ("full", (10158,)), ("full", (64, 225)), ("full", (5, 6, 7)), ("full", (3, 10007)),
+          ("dct", (4103,)), ("dct", (1021,)), ("dct", (20014,)), ("dct", (9, 10, 11)), ("dst", (999, 1000)),
+          ("dht", (33075,)), ("dht", (101, 6))]
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("kind,dims", SHARED)
+def test_two_streams_share_one_plan_forms(kind, dims, prec):
+    """Calls of one plan on distinct buffers alternate between two streams,
+    several deep; every result is to the last bit what the call gives alone."""
+    import torch
+    family = {"dct": "DCT", "dst": "DST", "dht": "DHT"}.get(kind, "FFT")
+    plan = getattr(jt, "%s%s_%dD" % ("Double" if prec == "f64" else "Float", family, len(dims)))(*dims)
+    names = {"c2c": ("complexForward", "complexInverse"), "real": ("realForward", "realInverse"),
+             "full": ("realForwardFull", "realInverseFull")}.get(kind, ("forward", "inverse"))
+    fwd, inv = (getattr(plan, m) for m in names)
+    if kind in ("dct", "dst"):
+        fwd = lambda a: plan.forward(a, True)  # noqa: E731
+    n = math.prod(dims) * (2 if kind in ("c2c", "full") else 1)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    dt = torch.float64 if prec == "f64" else torch.float32
+    src = [torch.randn(n, dtype=dt, device="cuda", generator=g) for _ in range(8)]
+    want = []
+    for i, x in enumerate(src):
+        y = x.clone()
+        inv(y, True) if i % 4 > 1 else fwd(y)
+        torch.cuda.synchronize()
+        want.append(y)
+    assert all(torch.isfinite(w).all() for w in want)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for rep in range(3):
+        bufs = [x.clone() for x in src]
+        torch.cuda.synchronize()
+        for i, b in enumerate(bufs):
+            with torch.cuda.stream(streams[i % 2]):
+                inv(b, True) if i % 4 > 1 else fwd(b)
+        torch.cuda.synchronize()
+        for i, b in enumerate(bufs):
+            assert torch.equal(b, want[i]), (rep, i)
+
+
 def test_threads_and_streams_mixed(orc):
     """Host-array calls from two threads while a third thread drives device
     calls on its own stream, all on one four-step plan."""
