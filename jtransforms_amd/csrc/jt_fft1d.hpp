@@ -701,7 +701,12 @@ inline void gen_set_shape(GenPlan& g, int W, bool col) {
 //   - at least one thread per 8 points: 3000 x 2000 FP32 148 against 164 with
 //     one per 16; one per 4 only while the chip is not full (360 x 640 26.5
 //     against 28.6, but 3000 x 2000 180).  Hooks have O(n) work of their own:
-//     up to one per 2 points there (DST 1000 x 1000 FP64 53 against 72).
+//     up to one per 2 points there (DST 1000 x 1000 FP64 53 against 72);
+//   - columns up to one thread per 2 points while there are under 2^16
+//     threads: the two passes of a four-step line are a few dozen workgroups,
+//     and a thread with several butterflies makes them one long chain (one
+//     c2c FP32 line of 16875 points 32.1 us against 28.9, of 78125 points 42.0
+//     against 36.2; up to 2^17 threads 720 x 1280 FP64 59 became 68).
 struct GenShape {
     int W, NT;
     size_t shm;
@@ -732,6 +737,8 @@ GenShape gen_shape(GenPlan& g, int64_t nlines, bool col, int eb, bool hooks) {
     // few lines: more threads per line hide more of each stage's latency
     const int most = std::min(1024, n * W / (hooks ? 2 : 4));
     while (2 * nt <= most && groups(W) * nt < (int64_t(1) << 18)) nt *= 2;
+    if (col && !hooks)
+        while (2 * nt <= std::min(1024, n * W / 2) && groups(W) * nt < (int64_t(1) << 16)) nt *= 2;
     if (!fits(W, 160 * 1024)) throw JtError(ST_UNSUPPORTED, "internal: length beyond the runtime-radix kernel");
     gen_set_shape(g, W, col);
     return GenShape{W, nt, bytes(W)};

@@ -119,6 +119,23 @@ def test_bluestein(orc, n, prec):
     assert rel(a, x) <= 2 * tol(6 * n, prec)
 
 
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("n", [8400, 13125, 16875, 27000, 33075, 78125, 192000])
+def test_four_step_few_lines(orc, n, prec):
+    """One line and a few of two passes of runtime-radix columns: up to one
+    thread per two points, with partly filled last workgroups."""
+    for lines in (1, 3):
+        x = orc.jrandom_doubles(n + lines, 2 * n * lines).astype(DT[prec])
+        p = jt.FFTBatch1D(n, lines, precision=prec)
+        a = x.copy()
+        p.complexForward(a)
+        for b in range(lines):
+            s = slice(2 * n * b, 2 * n * (b + 1))
+            assert rel(a[s], orc.complex_forward(n, x[s].astype(np.float64))) <= tol(n, prec), (lines, b)
+        p.complexInverse(a, True)
+        assert rel(a, x) <= 2 * tol(n, prec), lines
+
+
 # odd lengths (one launch; Bluestein in one launch; several launches), 2, and
 # even ones whose half has a large prime factor
 PAIR = [2, 3, 9, 37, 74, 225, 999, 1021, 2047, 4095, 4103, 10158]
