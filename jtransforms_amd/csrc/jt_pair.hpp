@@ -112,6 +112,14 @@ struct IOPair {
     }
     // forward: the outputs that Z_k and Z_{n-k} (k <= n/2; Z_0 twice for k = 0) give
     __device__ __forceinline__ void split(At at, I k, cpx<T> A, cpx<T> B, cpx<T> qk) const {
+        if constexpr (!paired) {
+            // Z_k = conj Z_{n-k} up to rounding, which their mean lowers by a
+            // quarter (halved first: the sum may be beyond the type's range)
+            const T h = T(0.5) * g;
+            wr(at, 2 * k == n ? 1 : 2 * k, A.x * h + B.x * h, T(0));
+            if (k > 0 && 2 * k != n) wr(at, 2 * k + 1 == n ? 1 : 2 * k + 1, A.y * h - B.y * h, T(0));
+            return;
+        }
         const cpx<T> Bc{B.x, -B.y};
         const cpx<T> s = cadd(A, Bc), d = csub(A, Bc);
         const T h = T(0.5) * g;
@@ -122,12 +130,9 @@ struct IOPair {
             const T f = k == 0 ? f0 : T(1);
             wr(at, sidx(k), a.x * f, b.x * f);
             if (k > 0 && 2 * k != n) wr(at, sidx(n - k), -a.y, -b.y);
-        } else if constexpr (KIND == R2R_DHT) {
+        } else {
             wr(at, k, a.x - a.y, b.x - b.y);
             if (k > 0 && 2 * k != n) wr(at, n - k, a.x + a.y, b.x + b.y);
-        } else {
-            wr(at, 2 * k == n ? 1 : 2 * k, a.x, b.x);
-            if (k > 0 && 2 * k != n) wr(at, 2 * k + 1 == n ? 1 : 2 * k + 1, a.y, b.y);
         }
     }
     // Both hooks take a few points at a time: all loads of a batch before its

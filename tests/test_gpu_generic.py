@@ -209,6 +209,19 @@ def test_packed_batch_lines_are_independent(orc, n, prec):
         assert not np.isfinite(y[1]).all() and not np.isfinite(y[2]).all(), op
 
 
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("n", [3, 225, 4095, 33075])
+def test_odd_packed_large_values(orc, n, prec):
+    """A sum of 0.6 times the type's largest value is a result, not an overflow."""
+    x = orc.jrandom_doubles(n, n) + 2.0  # positive: the first value is the largest
+    want = orc.real_forward(n, x)
+    top = 0.6 * float(np.finfo(DT[prec]).max) / np.abs(want).max()
+    a = (x * top).astype(DT[prec])
+    jt.FFTBatch1D(n, 1, precision=prec).realForward(a)
+    assert np.isfinite(a).all()
+    assert rel(a.astype(np.float64) / top, want) <= tol(n, prec)
+
+
 # single-launch, Bluestein and several-launch plans on each axis
 FULL = [(2,), (16,), (37,), (360,), (4096,), (2047,), (4103,), (10158,), (2, 2), (9, 37), (37, 16), (64, 225),
         (4103, 3), (3, 4103), (5, 6, 7), (16, 37, 9), (3, 4, 10158)]
