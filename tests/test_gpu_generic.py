@@ -257,18 +257,30 @@ def test_device_calls_after_the_first(orc):
     x = orc.jrandom_doubles(n, 2 * n + 3)
     p = jt.DoubleFFT_1D(n)
     want = orc.complex_forward(n, x[:2 * n])
-    s = torch.cuda.Stream()
     for rep in range(3):
         t = torch.from_numpy(x.copy()).cuda()
         torch.cuda.synchronize()
-        if rep == 2:
-            with torch.cuda.stream(s):
-                p.complexForward(t)
-            s.synchronize()
-        else:
-            p.complexForward(t)
+        p.complexForward(t)
         y = t.cpu().numpy()
         assert rel(y[:2 * n], want) <= tol(n, "f64") and np.array_equal(y[2 * n:], x[2 * n:])
+    # on a stream of the caller's: the input arrives there, behind work that
+    # takes milliseconds, so that a call on any other stream would transform
+    # what is in t before and then be overwritten
+    s = torch.cuda.Stream()
+    src = torch.from_numpy(x.copy()).cuda()
+    t = torch.zeros_like(src)
+    m = torch.ones(4096, 4096, device="cuda")
+    torch.mm(m, m)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        assert jt._raw_stream(torch, torch.cuda.current_device()) == s.cuda_stream
+        for _ in range(20):
+            torch.mm(m, m)
+        t.copy_(src)
+        p.complexForward(t)
+        y = t.to("cpu", non_blocking=False).numpy()
+    assert rel(y[:2 * n], want) <= tol(n, "f64")
+    assert jt._raw_stream(torch, torch.cuda.current_device()) == torch.cuda.current_stream().cuda_stream
     t = torch.from_numpy(x.copy()).cuda()
     p.complexForward(t, 3)  # misaligned pairs
     assert rel(t.cpu().numpy()[3:], orc.complex_forward(n, x[3:])) <= tol(n, "f64")

@@ -1,4 +1,5 @@
-"""Ragged batches (one persistent launch) against the oracle.
+"""Ragged batches (one persistent launch, or one launch per pass) against the
+oracle.
 Tolerances as for single transforms: FP64 rel-l2 <= 1e-13*log2(n), FP32
 <= 2e-7*log2(n) + 1e-6, per transform."""
 import math
@@ -58,6 +59,43 @@ def test_ragged_mixed(orc, prec, graph):
     for i, n in enumerate(lens):
         seg = slice(int(p.offsets[i]), int(p.offsets[i + 1]))
         assert rel(a[seg], x[seg]) <= 2 * tol(n, prec), n
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("graph", [False, True])
+def test_ragged_mixed_persistent(orc, prec, graph, monkeypatch):
+    """The same lengths (more points than the default's line) through the
+    persistent kernel, which smaller batches run: plain and as a captured graph,
+    forward and both inverses, replayed with eager work between."""
+    import torch
+    monkeypatch.setenv("JT_RAGGED_SCHEDULE", "form=persistent")
+    lens = np.array(MIXED, dtype=np.int64)
+    p = jt.RaggedBatch1D(lens, precision=prec, graph=graph)
+    assert "form=persistent" in p.describe()
+    x = orc.jrandom_doubles(20110602, int(2 * lens.sum())).astype(DT[prec])
+    want = [orc.complex_forward(int(n), x[int(p.offsets[i]):int(p.offsets[i + 1])].astype(np.float64))
+            for i, n in enumerate(lens)]
+    t = torch.from_numpy(x.copy()).cuda()
+    s = torch.cuda.Stream()
+    for rep in range(3 if graph else 1):  # graph: capture, then replays
+        out = []
+        with torch.cuda.stream(s):
+            t.copy_(torch.from_numpy(x))
+            p.complexForward(t)
+            y = t.clone()
+            out.append(y.cpu().numpy())
+            p.complexInverse(t, True)
+            out.append(t.cpu().numpy())
+            t.copy_(y)
+            p.complexInverse(t, False)
+            out.append(t.cpu().numpy())
+        s.synchronize()
+        p.sync_status()
+        for i, n in enumerate(lens):
+            seg = slice(int(p.offsets[i]), int(p.offsets[i + 1]))
+            assert rel(out[0][seg], want[i]) <= tol(n, prec), (rep, n)
+            assert rel(out[1][seg], x[seg]) <= 2 * tol(n, prec), (rep, n)
+            assert rel(out[2][seg], float(n) * x[seg].astype(np.float64)) <= 2 * tol(n, prec), (rep, n)
 
 
 @pytest.mark.parametrize("prec", ["f64", "f32"])
