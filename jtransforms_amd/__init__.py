@@ -233,7 +233,9 @@ class _Plan:
         if torch is not None and type(a) is torch.Tensor and a.is_cuda and a.dim() == 1 and a.is_contiguous():
             dev = a.get_device()
             need = self._elements.get(op)
-            if (need is not None and a.numel() - offa >= need and dev == torch.cuda.current_device()
+            if need is None:  # the plan's first call of op
+                need = self.elements(op)
+            if (a.numel() - offa >= need and dev == torch.cuda.current_device()
                     and a.dtype is (torch.float64 if self._precision == JT_F64 else torch.float32)):
                 rc = _lib.jt_execute(self._h, op, a.data_ptr(), offa, 1 if scale else 0, _raw_stream(torch, dev))
                 if rc:

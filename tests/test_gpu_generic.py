@@ -249,9 +249,29 @@ def test_real_full(orc, dims, prec):
         assert e <= tol(tot, prec), (fwd, e)
 
 
+@pytest.mark.parametrize("first", [True, False])
+def test_device_calls_refused(first):
+    """What a plan's calls on device tensors refuse, its first call or a later one."""
+    import torch
+    n = 600
+    good = torch.zeros(2 * n, dtype=torch.float64, device="cuda")
+    bad = [(TypeError, good.float()), (TypeError, good.cpu()), (TypeError, good.reshape(2, n)),
+           (TypeError, torch.zeros(4 * n, dtype=torch.float64, device="cuda")[::2]), (IndexError, good[:-1]),
+           (IndexError, good, 1), (ValueError, good, -1)]
+    for err, *args in bad:
+        p = jt.DoubleFFT_1D(n)
+        if not first:
+            p.complexForward(good)
+        with pytest.raises(err):
+            p.complexForward(*args)
+        p.complexForward(good)
+    with pytest.raises(ValueError):
+        jt.DoubleDCT_1D(n)._run(jt.COMPLEX_FORWARD, good)  # an op that the plan does not have
+
+
 def test_device_calls_after_the_first(orc):
-    """Later calls of a plan on flat device tensors take the short path: the
-    same results, streams, offsets and refusals as the first."""
+    """Calls of a plan on flat device tensors take a short path: the same
+    results, streams, offsets and refusals from the first call on."""
     import torch
     n = 600
     x = orc.jrandom_doubles(n, 2 * n + 3)
