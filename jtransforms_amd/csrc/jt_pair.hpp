@@ -96,7 +96,9 @@ struct IOPair {
                 u = cpx<T>{u.x * f0, u.y * f0};
                 w = cpx<T>{T(0), T(0)};
             }
-            // conj(q_k) (u - i w) of both lines, summed as A + i B
+            // half conj(q_k) (u - i w) of both lines, summed as A + i B
+            u = cpx<T>{u.x * T(0.5), u.y * T(0.5)};
+            w = cpx<T>{w.x * T(0.5), w.y * T(0.5)};
             return cmulc(cpx<T>{u.x + w.y, u.y - w.x}, q[k]);
         }
     }
@@ -120,10 +122,9 @@ struct IOPair {
             if (k > 0 && 2 * k != n) wr(at, 2 * k + 1 == n ? 1 : 2 * k + 1, A.y * h - B.y * h, T(0));
             return;
         }
-        const cpx<T> Bc{B.x, -B.y};
-        const cpx<T> s = cadd(A, Bc), d = csub(A, Bc);
-        const T h = T(0.5) * g;
-        cpx<T> a{s.x * h, s.y * h}, b{d.y * h, -d.x * h};  // g V_a, g V_b
+        const cpx<T> Ah{A.x * T(0.5), A.y * T(0.5)}, Bc{B.x * T(0.5), B.y * T(-0.5)};
+        const cpx<T> s = cadd(Ah, Bc), d = csub(Ah, Bc);
+        cpx<T> a{s.x * g, s.y * g}, b{d.y * g, -d.x * g};  // g V_a, g V_b
         if constexpr (makhoul) {
             a = cmul(qk, a);
             b = cmul(qk, b);

@@ -51,12 +51,15 @@ inline R2RScale dct3_scale(int64_t n, bool scale) {
 // ---------------------------------------------------------------------------
 template <int KIND, typename T>
 __device__ __forceinline__ void half_fwd(cpx<T> A, cpx<T> B, cpx<T> w, cpx<T> qa, cpx<T> qb, T* y) {
-    // A = Z_k, B = conj Z_{N-k}
+    // A = Z_k, B = conj Z_{N-k}; halved before they are summed, so that V_k up
+    // to the type's largest value does not overflow on the way
+    A = cpx<T>{A.x * T(0.5), A.y * T(0.5)};
+    B = cpx<T>{B.x * T(0.5), B.y * T(0.5)};
     const cpx<T> fe = cadd(A, B), d = csub(A, B);
     const cpx<T> fo = {d.y, -d.x};
     const cpx<T> wf = cmul(w, fo);
-    const cpx<T> Vk = {(fe.x + wf.x) * T(0.5), (fe.y + wf.y) * T(0.5)};
-    const cpx<T> Vc = {(fe.x - wf.x) * T(0.5), -(fe.y - wf.y) * T(0.5)};  // V_{N-k}
+    const cpx<T> Vk = {fe.x + wf.x, fe.y + wf.y};
+    const cpx<T> Vc = {fe.x - wf.x, -(fe.y - wf.y)};  // V_{N-k}
     if constexpr (KIND == R2R_DHT) {
         y[0] = Vk.x - Vk.y;
         y[1] = Vk.x + Vk.y;
@@ -343,7 +346,8 @@ __global__ void half_in(const T* __restrict__ x, cpx<T>* __restrict__ z, LineMap
             const T v0 = rd(j0), v1 = rd(j1);
             zl[k] = cpx<T>{KIND == R2R_DST && (j0 & 1) ? -v0 : v0, KIND == R2R_DST && (j1 & 1) ? -v1 : v1};
         } else {
-            auto a = [&](int64_t j) { return rd(KIND == R2R_DST ? n - 1 - j : j); };
+            // (halved: Z is then the result itself, not twice it)
+            auto a = [&](int64_t j) { return rd(KIND == R2R_DST ? n - 1 - j : j) * T(0.5); };
             if (k == 0) {
                 const T v0 = a(0) * f0, vN = T(1.41421356237309504880168872420970) * a(N);
                 zl[0] = cpx<T>{v0 + vN, v0 - vN};
@@ -511,8 +515,8 @@ void r2r_axis_k(const R2R1D<T>& r, T* data, LineMap lm, bool scale, cpx<T>* ws, 
         else run_single<T, (FWD || KIND == R2R_DHT) ? -1 : 1, true>(*r.half, io, st);
         return;
     }
-    // inverse: as above for the n-point and the half-length form alike
-    const T f0 = T(sc.f0), g = FWD || KIND == R2R_DHT ? T(sc.g) : T(sc.g * 0.5);
+    // (the n-point and the half-length form halve an inverse's inputs instead)
+    const T f0 = T(sc.f0), g = T(sc.g);
     const cpx<T>* q = r.q.template as<cpx<T>>();
     if (r.full) {
         pair_lines<T, KIND, FWD>(*r.full, data, q, lm, f0, g, ws, st);

@@ -222,6 +222,32 @@ def test_odd_packed_large_values(orc, n, prec):
     assert rel(a.astype(np.float64) / top, want) <= tol(n, prec)
 
 
+# line pairs of one launch and of several, half-length forms; (kind, n, forward, scale)
+LARGE = ([("dht", n, True, False) for n in (3, 225, 1021, 2042, 4103, 16875, 65536)]
+         + [("dct", n, True, False) for n in (3, 225, 1021, 4103, 10158)]
+         + [("dct", 3, False, True), ("dst", 3, False, True), ("dct", 65536, False, False),
+            ("dst", 65536, False, False)])
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("kind,n,fwd,scale", LARGE)
+def test_r2r_large_values(orc, kind, n, fwd, scale, prec):
+    """Results and inputs of up to 0.6 times the type's largest value."""
+    cls = {"dct": (jt.DoubleDCT_1D, jt.FloatDCT_1D), "dst": (jt.DoubleDST_1D, jt.FloatDST_1D),
+           "dht": (jt.DoubleDHT_1D, jt.FloatDHT_1D)}[kind][prec == "f32"]
+    x = orc.jrandom_doubles(n, n)
+    want = orc.realnd(kind, [n], x, fwd, scale)
+    top = 0.6 * float(np.finfo(DT[prec]).max) / max(np.abs(want).max(), np.abs(x).max())
+    a = (x * top).astype(DT[prec])
+    p = cls(n)
+    if fwd:
+        p.forward(a, *([scale] if kind != "dht" else []))
+    else:
+        p.inverse(a, scale)
+    assert np.isfinite(a).all()
+    assert rel(a.astype(np.float64) / top, want) <= tol(n, prec)
+
+
 # single-launch, Bluestein and several-launch plans on each axis
 FULL = [(2,), (16,), (37,), (360,), (4096,), (2047,), (4103,), (10158,), (2, 2), (9, 37), (37, 16), (64, 225),
         (4103, 3), (3, 4103), (5, 6, 7), (16, 37, 9), (3, 4, 10158)]
